@@ -239,8 +239,9 @@ int mxs_step(mxs_ctx* ctx, const mxs_batch* batch, const mxs_race* race, const m
 /* Candidates of the context's last mxs_sample or mxs_step call, per row of
  * its first `rows` rows, queued on the context's stream behind that call:
  * the list the row's finisher chose from (every candidate at or above its
- * chunk's threshold; it holds the row's top-k head for a top-k row and its
- * min-p set for a min-p row), as adjusted logits (penalties, bias, mask
+ * chunk's threshold; it holds the row's top-k head for a top-k row, its
+ * min-p set for a min-p row and, for a top-p row decided from its list, its
+ * nucleus), as adjusted logits (penalties, bias, mask
  * applied) with their token IDs, in token-ID order.  count[r] = the list's
  * length when at most `width`; else its top `width` by (logit desc, ID asc)
  * and count[r] = width; -1 for a row with no list (greedy, keep-all, error
@@ -316,7 +317,7 @@ enum {
   MXS_PATH_EXACT = 8,          /* working set in LDS, the nucleus certified without a sort */
   MXS_PATH_EXACT_SORTED = 9,   /* ... the crossing inside the min-p prefix: that prefix sorted */
   MXS_PATH_EXACT_REPLAY = 10,  /* ... an uncertain crossing: the reference's sums replayed */
-  MXS_PATH_LARGE = 11,         /* working set beyond LDS: mass-weighted radix select */
+  MXS_PATH_LARGE = 11,         /* working set beyond LDS (mass-weighted radix select), or a top-p row over its whole row */
   MXS_PATH_SHORT = 12          /* top-k <= 64 or min-p rows, at most 512 candidates: one wave, one E member per lane */
 };
 int mxs_debug_set_paths(mxs_ctx* ctx, void* device_buffer);

@@ -59,6 +59,7 @@ constexpr int MCAP = ((CHUNK_MAX / 32 + 2 + NT - 1) / NT) * NT;
 #define MXS_LA 3
 #endif
 constexpr int LA = MXS_LA;                // slices in flight ahead of pass 1 (lean chunk body)
+constexpr uint32_t NUC_MIN = 2048;        // a nucleus row's chunks list about this many tokens at least, together
 constexpr uint32_t WIDE_NCAND = 2048;     // a min-p chunk past this many candidates sums its mass in f64
 static_assert(HCAP % NT == 0 && BCAP % NT == 0 && MCAP % NT == 0,
               "LDS staging copies whole 1024-entry rounds");
@@ -220,6 +221,8 @@ struct alignas(16) FinSmem {
     uint32_t flags, nlegal, Mkey, bi, ncand;
     uint32_t qmax;                     // the largest candidate count of a chunk
     float lo;                          // no candidate is below it (the chunks' smallest threshold)
+    uint32_t tlo;                      // order key of the chunks' largest threshold (every legal token from it up is listed)
+    uint32_t st;                       // a nuc row's status
   } hdr;
   double etab[128];                    // exp_neg's tables: 2^(j/64) (high, low parts)
   double rd[FW][2];                    // multi-value reduction
@@ -323,6 +326,13 @@ __device__ __forceinline__ uint32_t chunk_mode(const RowCfg& c, uint32_t V) {
   return M_KEEPALL;
 }
 
+// Top-p alone (no active top-k, no min-p): the rows whose chunks list
+// nucleus candidates.  The other all-candidates rows (a top-k beyond
+// KCAND_MAX) list every legal token.
+__device__ __forceinline__ bool nucleus_only(const RowCfg& c, uint32_t V) {
+  return chunk_mode(c, V) == M_ALL && !(c.k > 0 && c.k < V);
+}
+
 // Logit-bias and penalty stage for one token (BUILD-DEFINED semantics, f32,
 // every operation rounded separately).
 __device__ __forceinline__ float adjust(float l, uint32_t cnt, uint32_t slot, float bias, const RowCfg& c) {
@@ -412,6 +422,8 @@ struct FinCtx {
   double M, L, Lclose, total, total_err;
   bool have_total;
   bool nodraw;         // race-v2: the draw is discarded, so only the kept set's certificate sets the status
+  bool nuc;            // a top-p row over its chunks' nucleus candidates (status 1: finished over the whole row instead)
+  uint32_t* stw;       // the status written last, for nuc rows (LDS)
   uint32_t* kbits;
   uint32_t nwords;
   uint64_t* timing;    // phase timestamps (diagnostics), null when off
@@ -462,6 +474,7 @@ __device__ __forceinline__ void write_result(const FinCtx& X, int32_t status, in
     const mxs_out& o = X.o;
     o.token[X.row] = token;
     o.status[X.row] = status;
+    if (X.nuc) *X.stw = (uint32_t)status;
     if (o.sampling_logprob) o.sampling_logprob[X.row] = lp;
     if (o.kept_count) o.kept_count[X.row] = kept;
   }
@@ -2977,7 +2990,9 @@ __device__ __forceinline__ bool finish_w1(const FinCtx& X, FinSmem& F) {
   } else if (c.top_p < 1.0) {
     // the reference walks the tokens whose weight reaches 1e-9 of the total:
     // every min-p member must clear that level
-    if (!(c.min_p * (1.0 - 1e-12) > 1e-9 * (X.total + X.total_err) * (1.0 + 1e-12))) return false;
+    // (a nuc row's cut is known to lie among its candidates; below the 1e-9
+    // level the reference falls back to the whole row, the same prefix)
+    if (!X.nuc && !(c.min_p * (1.0 - 1e-12) > 1e-9 * (X.total + X.total_err) * (1.0 + 1e-12))) return false;
     theta_set = true;
     theta = c.top_p * X.total;
     theta_err = c.top_p * X.total_err + U * theta;
@@ -3223,9 +3238,13 @@ __device__ __forceinline__ uint32_t reduce_head(const float* cand_l, const uint3
   return res;
 }
 
+// `nuc_row`: a top-p row (no top-k, no min-p) whose chunks listed their nucleus
+// candidates and their whole mass; returns true when the row has to be
+// finished over every legal token instead (the nucleus may reach below what
+// every chunk lists, or the f32 part of the mass left a cut uncertified).
 template <typename In>
-__device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, const RowCfg& c, uint32_t row, uint32_t mode,
-                           uint64_t rbase, double invT, const FinLoads& P) {
+__device__ __forceinline__ bool finish_row(const SampleArgs& A, FinSmem& F, const RowCfg& c, uint32_t row, uint32_t mode,
+                           uint64_t rbase, double invT, const FinLoads& P, const bool nuc_row) {
   const mxs_batch& b = A.b;
   const uint32_t tid = threadIdx.x;
   const uint32_t V = b.vocab;
@@ -3260,6 +3279,7 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
     const uint32_t qmax = wave_max_u32(v.ncand);
     // the smallest candidate threshold (order keys; chunks without candidates do not count)
     const uint32_t lokey = ~wave_max_u32(v.ncand ? ~okey(v.thr) : 0u);
+    const uint32_t tlo = nuc_row ? wave_max_u32(v.nlegal ? okey(v.thr) : 0u) : 0u;
     // the greedy argmax: largest (value key, ~id); chunk values are +0.0-normalised
     const unsigned long long garg = wave_max_u64(
         v.gbest_id != NONE ? ((unsigned long long)okey(v.gbest_val) << 32) | (unsigned long long)(~v.gbest_id) : 0ull);
@@ -3279,6 +3299,7 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
       // token's f32::MIN would otherwise stretch the bins over 3.4e38 and
       // put every other candidate in bin 0).
       F.hdr.lo = fmaxf(okey_value(lokey), okey_value(mkey) - (float)(746.0 * c.T));
+      F.hdr.tlo = tlo;
     }
   } else if (wave() == 1 && !c.greedy) {
     // the chunk masses rescaled to the row maximum (f64: off wave 0's path)
@@ -3310,19 +3331,24 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
   X.cand_l = A.w.cand_l; X.cand_id = A.w.cand_id; X.CH = A.CH; X.o = A.o; X.c = c; X.row = row; X.mode = mode; X.C = C; X.V = V; X.nlegal = nlegal; X.rbase = rbase;
   X.kbits = kbits; X.nwords = nwords; X.M = M; X.timing = A.timing; X.paths = A.paths; X.etab = F.etab;
   X.nodraw = A.nodraw != 0u;
+  // (chunks that list every legal token: their sum is the row's, as for any
+  // all-candidates row)
+  const bool nuc = nuc_row && okey_value(F.hdr.tlo) > -INFINITY;
+  X.nuc = nuc;
+  X.stw = &F.hdr.st;
   if (err) {
     fpath(X, MXS_PATH_ERROR);
     write_result(X, err, -1, 0.0, 0u);
     if (kbits)
       for (uint32_t q = tid; q < nwords; q += FT) kbits[q] = 0u;
-    return;
+    return false;
   }
   if (mode == M_GREEDY) {
     fpath(X, MXS_PATH_GREEDY);
     write_result(X, 0, (int32_t)bi, 0.0, 1u);
     if (kbits)
       for (uint32_t q = tid; q < nwords; q += FT) kbits[q] = (q == (bi >> 5)) ? (1u << (bi & 31u)) : 0u;
-    return;
+    return false;
   }
   const bool k_act = c.k > 0 && c.k < nlegal;
 
@@ -3331,12 +3357,12 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
     uint32_t mink = NONE;
     for (uint32_t q = 0; q < C; ++q)
       if (F.st[q].nlegal && F.st[q].minkey < mink) mink = F.st[q].minkey;
-    if (!isfinite(((double)okey_value(mink) - M) / c.T)) { write_result(X, MXS_ROW_INVALID_TEMPERATURE, -1, 0.0, 0u); return; }
+    if (!isfinite(((double)okey_value(mink) - M) / c.T)) { write_result(X, MXS_ROW_INVALID_TEMPERATURE, -1, 0.0, 0u); return false; }
     if (A.nodraw) {   // race-v2: the kept set is every legal token; the race kernel picks
       fpath(X, MXS_PATH_KEEPALL_RACE);
       write_result(X, 0, -1, 0.0, nlegal);
       keepall_bits(A, row, kbits, nwords, V);
-      return;
+      return false;
     }
     fpath(X, MXS_PATH_KEEPALL);
     const uint32_t segs_per_chunk = A.per * NW;   // the chunk kernel's 256-token (slice, wave) segments
@@ -3386,7 +3412,7 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
       near = true;
       before = -INFINITY;   // forces the last positive token of the segment
     }
-    if (seg == NONE) { write_result(X, MXS_ROW_EMPTY_SUPPORT, -1, 0.0, 0u); return; }
+    if (seg == NONE) { write_result(X, MXS_ROW_EMPTY_SUPPORT, -1, 0.0, 0u); return false; }
     if (wave() == 0) {
       const uint32_t q = seg / segs_per_chunk, r = seg % segs_per_chunk;
       const uint32_t i = r / NW, w = r % NW;
@@ -3458,11 +3484,11 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
     }
     __syncthreads();
     const uint32_t tok = F.s_u[3];
-    if (tok == NONE) { write_result(X, MXS_ROW_EMPTY_SUPPORT, -1, 0.0, 0u); return; }
+    if (tok == NONE) { write_result(X, MXS_ROW_EMPTY_SUPPORT, -1, 0.0, 0u); return false; }
     near = near || F.s_u[4] != 0u;
     write_result(X, near ? MXS_ROW_UNCERTIFIED : 0, (int32_t)tok, F.s_d[1] - log(total), nlegal);
     keepall_bits(A, row, kbits, nwords, V);
-    return;
+    return false;
   }
 
   // =================== candidate paths ====================================
@@ -3498,7 +3524,7 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
   X.have_total = false;
   // (an all-candidates row's working set is every legal token: its sum is
   // the total)
-  if (c.top_p < 1.0 && !k_act && (mode == M_MINP || (mode == M_TOPK && A.masked))) {
+  if (c.top_p < 1.0 && !k_act && (mode == M_MINP || (mode == M_TOPK && A.masked) || nuc)) {
     X.total = F.hdr.mass;
     X.total_err = F.hdr.mass_err;
     X.have_total = true;
@@ -3549,12 +3575,38 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
     }
     lds_barrier();
   };
-  // short rows first: the one-wave finisher
   bool loaded = pre;
-  if (((mode == M_TOPK && c.k <= 64u) || mode == M_MINP) && ncand > 0u && ncand <= (uint32_t)(WR * 64) &&
-      X.lds_c) {
+  // the status thread 0 wrote for a nuc row, seen by the workgroup
+  auto nuc_open = [&]() -> bool {
+    __syncthreads();
+    return F.hdr.st == (uint32_t)MXS_ROW_UNCERTIFIED;
+  };
+  // A nuc row: the nucleus lies among the candidates every chunk lists in
+  // full (those from the largest chunk threshold up) when their mass reaches
+  // top_p of the row's.  f32 weights: relative error below 1e-5 (three
+  // roundings of an exponent of at most 126 octaves and 2 ulp of exp2); a
+  // mass within 4e-5 of the bar counts as below it.
+  if (nuc_row && !X.lds_c) return true;
+  const bool short_row = ((mode == M_TOPK && c.k <= 64u) || mode == M_MINP) && ncand > 0u &&
+                         ncand <= (uint32_t)(WR * 64) && X.lds_c;
+  if (short_row || nuc) {
     if (!loaded) bulk_load();
     loaded = true;
+  }
+  if (nuc) {
+    const float Mf = (float)M, c2 = (float)(invT * 1.4426950408889634), tl = okey_value(F.hdr.tlo);
+    float z = 0.0f;
+#pragma unroll
+    for (int u = 0; u < FR; ++u) {
+      const uint32_t j = (uint32_t)u * FT + tid;
+      const float l = j < ncand ? F.cl[j] : -INFINITY;
+      z += l >= tl && j < ncand ? __builtin_amdgcn_exp2f((l - Mf) * c2) : 0.0f;
+    }
+    const double Z = block_sum<double>((double)z, F.red_d);
+    if (!(Z * (1.0 - 4e-5) >= c.top_p * (X.total + X.total_err))) return true;
+  }
+  // short rows first: the one-wave finisher
+  if (short_row) {
     if (wave() == 0) {
       const bool ok = finish_w1(X, F);
       if (lane() == 0) F.s_u[15] = ok ? 1u : 0u;
@@ -3563,7 +3615,7 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
     if (F.s_u[15]) {
       fpath(X, MXS_PATH_SHORT);
       stamp(A, row, MAXC, 2);
-      return;
+      return false;
     }
     lds_barrier();   // wave 0's LDS scratch is reused below
   }
@@ -3572,7 +3624,7 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
     if (finish_sel(X, F, P, sq, sj)) {
       fpath(X, MXS_PATH_SELECT);
       stamp(A, row, MAXC, 2);
-      return;
+      return false;
     }
   }
   if (X.lds_c && !loaded) bulk_load();
@@ -3587,14 +3639,14 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
     if (F.s_u[15]) {
       fpath(X, MXS_PATH_WAVE);
       stamp(A, row, MAXC, 2);
-      return;
+      return nuc && nuc_open();
     }
     lds_barrier();   // wave 0's LDS scratch is reused below
   }
   if (mode != M_KEEPALL && finish_fast(X, F)) {
     fpath(X, MXS_PATH_FAST);
     stamp(A, row, MAXC, 2);
-    return;
+    return nuc && nuc_open();
   }
   __syncthreads();   // the general path below reuses LDS the lean finisher touched
   uint32_t ties_needed = 0;
@@ -3736,6 +3788,365 @@ __device__ __forceinline__ void finish_row(const SampleArgs& A, FinSmem& F, cons
     if (X.lds_c) finish_large_r(X, F, ne);
     else finish_large(X, F, ne);
     if (mp_close && tid == 0 && A.o.status[row] == 0) A.o.status[row] = MXS_ROW_UNCERTIFIED;
+  }
+  return nuc && nuc_open();
+}
+
+// ---------------------------------------------------------------------------
+// The nucleus of a whole row on one workgroup: top-p rows whose chunks'
+// candidates did not decide it (nuclei of many thousands of tokens, or a cut
+// inside the candidates' error bound).  Wave w reads the quads from w QW on,
+// 64 per step, so (wave, step) order is token-ID order:
+//   1  f64 weights onto NB mass bins of 1/64 octave below the row maximum;
+//      the prefix over the bins finds the one where the mass reaches theta
+//   2  that bin's members sorted by (key desc, ID asc) when ECAP hold them,
+//      after mass histograms on their keys while they don't; equal keys
+//      beyond that are cut by their count
+//   3  the kept tokens' mass per segment of `g` steps, then one wave draws
+//      inside the segment that holds the variate.
+// Every comparison carries the error bound of the f64 sums; one inside it
+// reports the row uncertified.  Bound by one workgroup's f64 arithmetic:
+// about 55 operations per weight and 150 weights per thread and pass.
+template <typename In>
+__device__ __forceinline__ void finish_nuc(const SampleArgs& A, FinSmem& F, const RowCfg& c, uint32_t row, double invT) {
+  const mxs_batch& b = A.b;
+  const uint32_t tid = threadIdx.x, V = b.vocab, nq = (V + 3u) / 4u;
+  const uint32_t QW = ((nq + (uint32_t)FW - 1u) / (uint32_t)FW + 63u) & ~63u, nj = QW / 64u, q0 = wave() * QW + lane();
+  const bool dense = c.he > c.hb || c.be > c.bb, masked = A.masked != 0u;
+  const uint32_t lim = masked ? min(V, b.tokenizer_vocab) : V;
+  const In* src = reinterpret_cast<const In*>(b.logits) + (uint64_t)row * b.row_stride;
+  const uint2* adj = reinterpret_cast<const uint2*>(A.w.adj + (uint64_t)row * ((V + 3u) & ~3u));
+  const uint32_t* mw = b.mask_words + (uint64_t)row * b.mask_stride;
+  const uint32_t nlegal = F.hdr.nlegal;
+  const float Mf = okey_value(F.hdr.Mkey);
+  const double M = (double)Mf;
+  const float hs = (float)(invT * 1.4426950408889634) * 64.0f;
+  auto weight = [&](float l) { return exp_neg_t(((double)l - M) / c.T, F.etab, F.etab + 64); };
+  auto bin_of = [&](float l) { return (uint32_t)fminf((Mf - l) * hs, (float)(NB - 1)); };
+  // quad q's first token ID, adjusted logits and legal bits
+  auto load_quad = [&](uint32_t q, uint32_t* id0, float* x) -> uint32_t {
+    const uint32_t e0 = 4u * q, qs = e0 < lim ? q : 0u;
+    *id0 = e0;
+    if (dense) {
+      const uint2 a = ld_dev(adj + 2u * qs), d = ld_dev(adj + 2u * qs + 1u);
+      x[0] = __uint_as_float(a.x); x[1] = __uint_as_float(a.y);
+      x[2] = __uint_as_float(d.x); x[3] = __uint_as_float(d.y);
+    } else {
+      Quad<In>::unpack(Quad<In>::load(src + 4u * qs), x);
+    }
+    uint32_t m = e0 < lim ? (lim - e0 >= 4u ? 0xfu : (1u << (lim - e0)) - 1u) : 0u;
+    if (masked) m &= mw[qs >> 3] >> ((qs & 7u) * 4u);
+    return m;
+  };
+  // one pass over the row: f(step, first token ID, logits, legal bits)
+  auto each = [&](auto f) {
+    constexpr int UN = 2;   // quads in flight per thread
+    for (uint32_t j = 0; j < nj; j += UN) {
+      float x[UN][4];
+      uint32_t lb[UN], id[UN];
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {
+        lb[u] = load_quad(q0 + (j + (uint32_t)u) * 64u, &id[u], x[u]);
+        if (j + (uint32_t)u >= nj) lb[u] = 0u;   // the next wave's
+      }
+#pragma unroll
+      for (int u = 0; u < UN; ++u) f(j + (uint32_t)u, id[u], x[u], lb[u]);
+    }
+  };
+  // |a computed sum of n weights - the reference's|
+  auto bound = [&](double v, uint32_t n) { return sum_bound(v, n + 64u, 8.0); };
+  bool uncert = false;
+  if (A.paths && tid == 0) A.paths[row] = MXS_PATH_LARGE;
+
+  // ---- 1: the mass bins ----------------------------------------------------
+  uint32_t* hc = F.u.h.hcnt;
+  double* hm = F.u.h.hmass;
+  auto clear_bins = [&]() {
+    for (uint32_t t = tid; t < (uint32_t)NB; t += FT) { hc[t] = 0u; hm[t] = 0.0; }
+    if (tid == 0) { F.s_u[4] = NONE; F.s_u[6] = 0u; F.s_u[8] = 0u; }
+    __syncthreads();
+  };
+  double above = 0.0, theta = 0.0, theta_err = 0.0;   // mass ranked before the bin
+  uint32_t above_n = 0, members = 0;
+  // the bin where the prefix reaches theta, bin 0 first; the first pass also
+  // sums the row (total) and sets theta
+  auto cross = [&](bool first) -> uint32_t {
+    __syncthreads();
+    const uint32_t b0 = 2u * tid;
+    const double v0 = hm[b0], v1 = hm[b0 + 1u];
+    const uint32_t n0 = hc[b0], n1 = hc[b0 + 1u];
+    double exc, tot;
+    uint32_t nin, ntot;
+    const double inc = block_scan_pair_du(v0 + v1, n0 + n1, F.red_d, F.red_u, &exc, &tot, &nin, &ntot);
+    if (first) {
+      theta = c.top_p * tot;
+      theta_err = c.top_p * bound(tot, nlegal) + U * theta;
+    }
+    double lo = above + exc;
+    uint32_t nlo = above_n + nin - n0 - n1;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t nh = i ? n1 : n0;
+      const double hi = i ? above + inc : lo + v0;
+      if (nh && lo < theta && theta <= hi) {
+        F.s_u[4] = b0 + (uint32_t)i; F.s_u[5] = nlo; F.s_u[7] = nh; F.s_d[4] = lo;
+        if (!(lo + bound(lo, nlo) < theta - theta_err) || !(hi - bound(hi, nlo + nh) >= theta + theta_err)) F.s_u[6] = 1u;
+      }
+      lo = hi;
+      nlo += nh;
+    }
+    __syncthreads();
+    const uint32_t bin = F.s_u[4];
+    if (bin != NONE) {
+      if (F.s_u[6]) uncert = true;
+      above = F.s_d[4];
+      above_n = F.s_u[5];
+      members = F.s_u[7];
+    }
+    __syncthreads();
+    return bin;
+  };
+  clear_bins();
+  each([&](uint32_t, uint32_t, const float* x, uint32_t lb) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if ((lb >> e) & 1u) {
+        const uint32_t t = bin_of(x[e]);
+        atomicAdd(&hc[t], 1u);
+        atomicAdd(&hm[t], weight(x[e]));
+      }
+  });
+  const uint32_t bin = cross(true);
+  // ---- 2: the cut inside the bin --------------------------------------------
+  uint32_t cut_key = 0u, cut_id = NONE;   // kept: a larger key, or the cut's and an ID up to cut_id
+  if (bin == NONE) {
+    uncert = true;   // rounding left theta past the row's mass: everything is kept
+  } else {
+    uint32_t klo = 0u, khi = NONE;   // the members' key range
+    auto member_key = [&](float l, uint32_t* k) { *k = okey(l); return bin_of(l) == bin && *k >= klo && *k <= khi; };
+    while (members > (uint32_t)ECAP && klo != khi) {
+      // a crowded bin: its keys' range, then the mass on NB bins of that range
+      uint32_t kmn = NONE, kmx = 0u, k;
+      each([&](uint32_t, uint32_t, const float* x, uint32_t lb) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (((lb >> e) & 1u) && member_key(x[e], &k)) { kmn = min(kmn, k); kmx = max(kmx, k); }
+      });
+      khi = block_max<uint32_t>(kmx, F.red_u);
+      klo = ~block_max<uint32_t>(~kmn, F.red_u);
+      if (klo == khi) break;
+      const uint32_t span = khi - klo;
+      const int sh = max(0, 32 - (int)__clz((int)span) - 11);   // span >> sh < NB
+      clear_bins();
+      each([&](uint32_t, uint32_t, const float* x, uint32_t lb) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (((lb >> e) & 1u) && member_key(x[e], &k)) {
+            const uint32_t t = (khi - k) >> sh;
+            atomicAdd(&hc[t], 1u);
+            atomicAdd(&hm[t], weight(x[e]));
+          }
+      });
+      const uint32_t t = cross(false);
+      if (t == NONE) { uncert = true; break; }
+      const uint32_t top = khi - (t << sh);
+      khi = top;
+      klo = max(klo, top - ((1u << sh) - 1u));
+    }
+    if (members <= (uint32_t)ECAP) {
+      uint32_t k;
+      if (tid == 0) { F.s_u[8] = 0u; F.s_u[6] = NONE; F.s_u[7] = 0u; }
+      __syncthreads();
+      each([&](uint32_t, uint32_t id0, const float* x, uint32_t lb) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (((lb >> e) & 1u) && member_key(x[e], &k)) {
+            const uint32_t at = atomicAdd(&F.s_u[8], 1u);
+            if (at < (uint32_t)ECAP) F.u.e.skey[at] = ((unsigned long long)k << 32) | (unsigned long long)(~(id0 + (uint32_t)e));
+          }
+      });
+      __syncthreads();
+      const uint32_t nm = min(F.s_u[8], (uint32_t)ECAP);
+      bitonic_sort_desc(F.u.e.skey, nm);
+      double run = above;
+      for (uint32_t base = 0; base < nm; base += FT) {
+        const uint32_t p = base + tid;
+        const double w = p < nm ? weight(okey_value((uint32_t)(F.u.e.skey[p] >> 32))) : 0.0;
+        double exc, tot;
+        const double inc = run + block_scan_pair<double>(w, F.red_d, &exc, &tot);
+        exc += run;
+        if (p < nm && inc >= theta && (exc < theta || p == 0u)) {
+          F.s_u[6] = p;
+          if (!(inc - bound(inc, above_n + p + 1u) >= theta + theta_err) || !(exc + bound(exc, above_n + p) < theta - theta_err))
+            F.s_u[7] = 1u;
+        }
+        run += tot;
+      }
+      __syncthreads();
+      const uint32_t at = F.s_u[6] == NONE ? nm - 1u : F.s_u[6];
+      if (F.s_u[7] || F.s_u[6] == NONE) uncert = true;
+      cut_key = (uint32_t)(F.u.e.skey[at] >> 32);
+      cut_id = ~(uint32_t)F.u.e.skey[at];
+    } else {
+      // equal keys: the first `need` of them in token-ID order are kept
+      cut_key = klo;
+      const double wt = weight(okey_value(klo));
+      const double steps = wt > 0.0 ? ceil((theta - above) / wt) : 1.0;
+      const uint32_t need = steps >= 1.0 ? (steps < (double)members ? (uint32_t)steps : members) : 1u;
+      const double hi = above + wt * (double)need, lo = hi - wt;
+      const double eb = bound(hi, above_n + need) + theta_err;
+      if (!(hi - eb >= theta) || (need > 1u && !(lo + eb < theta))) uncert = true;
+      uint32_t mine = 0u;   // this wave's members
+      each([&](uint32_t, uint32_t, const float* x, uint32_t lb) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          mine += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(((lb >> e) & 1u) && okey(x[e]) == klo));
+      });
+      if (lane() == 0) F.ru[wave()][0] = mine;
+      if (tid == 0) F.s_u[8] = NONE;
+      __syncthreads();
+      uint32_t seen = 0u;
+      for (uint32_t w = 0; w < wave(); ++w) seen += F.ru[w][0];
+      each([&](uint32_t, uint32_t id0, const float* x, uint32_t lb) {
+        uint32_t tb = 0u;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tb |= ((lb >> e) & 1u) && okey(x[e]) == klo ? 1u << e : 0u;
+        const uint32_t n = (uint32_t)__builtin_popcount(tb), inc = wave_scan_u32(n);
+        uint32_t r = seen + inc - n;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if ((tb >> e) & 1u) { ++r; if (r == need) F.s_u[8] = id0 + (uint32_t)e; }
+        seen += bcast63(inc);
+      });
+      __syncthreads();
+      cut_id = F.s_u[8];
+    }
+  }
+  __syncthreads();
+
+  // ---- 3: the kept tokens' mass, and the draw -------------------------------
+  constexpr uint32_t SEGS = (uint32_t)CCAP / FW;   // segments per wave (sums over the candidate cache)
+  double* seg = reinterpret_cast<double*>(F.cl);
+  static_assert(offsetof(FinSmem, cid) == offsetof(FinSmem, cl) + CCAP * 4, "the sums take cl and cid");
+  const uint32_t g = (nj + SEGS - 1u) / SEGS, ns = (nj + g - 1u) / g;
+  auto kept_of = [&](float l, uint32_t id) { const uint32_t k = okey(l); return k > cut_key || (k == cut_key && id <= cut_id); };
+  uint32_t* kbits = A.o.kept_bits ? A.o.kept_bits + (uint64_t)row * ((V + 31u) / 32u) : nullptr;
+  double part = 0.0;
+  uint32_t kn = 0u, bad = 0u, filled = 0u, at_seg = 0u;
+  each([&](uint32_t j, uint32_t id0, const float* x, uint32_t lb) {
+    uint32_t kb = 0u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (((lb >> e) & 1u) && kept_of(x[e], id0 + (uint32_t)e)) {
+        kb |= 1u << e;
+        part += weight(x[e]);
+        if (!isfinite(((double)x[e] - M) / c.T)) bad = 1u;
+      }
+    kn += (uint32_t)__builtin_popcount(kb);
+    if (kbits) {   // eight lanes' nibbles make a word
+      uint32_t w = kb << ((lane() & 7u) * 4u);
+      w |= (uint32_t)__shfl_xor((int)w, 1);
+      w |= (uint32_t)__shfl_xor((int)w, 2);
+      w |= (uint32_t)__shfl_xor((int)w, 4);
+      if ((lane() & 7u) == 0u && j < nj && id0 < V) kbits[id0 >> 5] = w;
+    }
+    if (j < nj && ++filled == g) {
+      const double ws = wave_sum_f64(part);
+      if (lane() == 0) seg[wave() * ns + at_seg] = ws;
+      ++at_seg;
+      filled = 0u;
+      part = 0.0;
+    }
+  });
+  if (filled) {
+    const double ws = wave_sum_f64(part);
+    if (lane() == 0) seg[wave() * ns + at_seg] = ws;
+  }
+  if (block_max<uint32_t>(bad, F.red_u)) {
+    if (tid == 0) {
+      A.o.token[row] = -1;
+      A.o.status[row] = MXS_ROW_INVALID_TEMPERATURE;
+      if (A.o.sampling_logprob) A.o.sampling_logprob[row] = 0.0;
+      if (A.o.kept_count) A.o.kept_count[row] = 0u;
+    }
+    return;
+  }
+  const uint32_t nkept = block_sum<uint32_t>(kn, F.red_u);
+  const uint32_t nseg = ns * (uint32_t)FW, per = (nseg + FT - 1u) / FT, s0 = tid * per;
+  double sp = 0.0;
+  for (uint32_t i = 0; i < per; ++i)
+    if (s0 + i < nseg) sp += seg[s0 + i];
+  double exc, S;
+  const double inc = block_scan_pair<double>(sp, F.red_d, &exc, &S);
+  const double target = c.u * S, derr = bound(S, nkept);
+  if (tid == 0) { F.s_u[0] = NONE; F.s_u[1] = 0u; F.s_u[3] = NONE; F.s_u[4] = 1u; }
+  __syncthreads();
+  {
+    double cum = exc;
+    uint32_t lastp = 0u;
+    for (uint32_t i = 0; i < per; ++i) {
+      if (s0 + i >= nseg) break;
+      const double w = seg[s0 + i], prev = cum;
+      cum = i + 1u == per ? inc : cum + w;
+      if (w > 0.0) lastp = s0 + i + 1u;
+      if (w > 0.0 && target < cum && !(target < prev)) { F.s_u[0] = s0 + i; F.s_d[0] = prev; }
+    }
+    const uint32_t lp = wave_max_u32(lastp);
+    if (lane() == 0 && lp) atomicMax(&F.s_u[1], lp);
+  }
+  __syncthreads();
+  const bool hit = F.s_u[0] != NONE;
+  const uint32_t sg = hit ? F.s_u[0] : F.s_u[1] - 1u;   // rounding past the mass: the last positive segment
+  if ((hit || F.s_u[1]) && wave() == 0) {
+    const uint32_t sw = sg / ns, sj = sg % ns;
+    double run = hit ? F.s_d[0] : 0.0;
+    uint32_t last = 0u;   // this lane's last positive token, ID + 1
+    float lastl = 0.0f;
+    for (uint32_t i = 0; i < g; ++i) {
+      const uint32_t j = sj * g + i;
+      if (j >= nj) break;
+      float x[4];
+      uint32_t e0;
+      const uint32_t lb = load_quad(sw * QW + j * 64u + lane(), &e0, x);
+      double w[4], ls = 0.0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        w[e] = ((lb >> e) & 1u) && kept_of(x[e], e0 + (uint32_t)e) ? weight(x[e]) : 0.0;
+        ls += w[e];
+      }
+      const double li = wave_scan_f64(ls);
+      double cum = run + (li - ls);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const double prev = cum;
+        cum += w[e];
+        if (!(w[e] > 0.0)) continue;
+        last = e0 + (uint32_t)e + 1u;
+        lastl = x[e];
+        if (hit && target < cum && !(target < prev)) {
+          F.s_u[3] = e0 + (uint32_t)e;
+          F.s_d[1] = ((double)x[e] - M) / c.T;
+          F.s_u[4] = fabs(target - prev) <= derr || fabs(cum - target) <= derr ? 1u : 0u;
+        }
+      }
+      run += bcast63(li);
+    }
+    wave_lds_sync();
+    const uint32_t lm = wave_max_u32(last);
+    if (F.s_u[3] == NONE && last == lm && lm) {   // past the accumulated mass: the last positive token, uncertified
+      F.s_u[3] = lm - 1u;
+      F.s_d[1] = ((double)lastl - M) / c.T;
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    const uint32_t tok = F.s_u[3];
+    const bool none = tok == NONE;
+    if (F.s_u[4] && !A.nodraw) uncert = true;
+    A.o.token[row] = none ? -1 : (int32_t)tok;
+    A.o.status[row] = none ? MXS_ROW_EMPTY_SUPPORT : (uncert ? MXS_ROW_UNCERTIFIED : 0);
+    if (A.o.sampling_logprob) A.o.sampling_logprob[row] = none ? 0.0 : F.s_d[1] - log(S);
+    if (A.o.kept_count) A.o.kept_count[row] = none ? 0u : nkept;
   }
 }
 
@@ -4915,7 +5326,11 @@ __device__ __forceinline__ uint32_t chunk_fast(const SampleArgs& A, FusedSmem& U
 // already read the row's parameters (c).  The kernel's own load of the
 // first slice is not passed in (it would stay live across both bodies): the
 // general body issues its slices itself.
-template <typename In>
+// NUC: the body of the nucleus-only rows (top-p alone, no parameter error).
+// A separate instantiation: with the nucleus threshold in it, the body for
+// the other rows spilled (56 registers; grammar-masked bf16 rows 43 -> 55 us
+// per call).
+template <typename In, bool NUC>
 __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem& U, const RowCfg& c,
                                               const uint32_t row, const uint32_t chunk, const bool rx) {
   ChunkSmem& S = chunk_smem(U);
@@ -4936,7 +5351,7 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
   // first quad is re-read and ignored.
   typename Quad<In>::Raw raw[PER_MAX];
   raw[0] = Quad<In>::load(src + (c0 + tid * 4u < c1 ? c0 + tid * 4u : c0));
-  const uint32_t mode = chunk_mode(c, V);
+  const uint32_t mode = NUC ? (uint32_t)M_ALL : chunk_mode(c, V);
   const double invT = c.greedy ? 0.0 : 1.0 / c.T;
   const uint32_t hn = c.he > c.hb ? c.he - c.hb : 0u, bn = c.be > c.bb ? c.be - c.bb : 0u;
   const bool has_tab = hn || bn;
@@ -4975,6 +5390,14 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
     const uint32_t e0 = c0 + (uint32_t)i * SLICE + tid * 4u;
     raw[i] = Quad<In>::load(src + (e0 < c1 ? e0 : c0));
   }
+  // T ln(V / (1 - top_p)): tokens further than this below the row maximum
+  // weigh less than (1 - top_p) / V of the total each, so all of them
+  // together stay outside the nucleus (taken while the loads are in flight)
+  double nuc_reach = 0.0;
+  if constexpr (NUC) {
+    nuc_reach = c.T * log((double)V / (1.0 - c.top_p));
+    __asm__ volatile("" : "+v"(nuc_reach));
+  }
   if (stage_h) {
 #pragma unroll
     for (int r = 0; r < HCAP / NT; ++r) S.hids[r * NT + tid] = hreg[r];
@@ -4999,7 +5422,7 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
   } else if (tab_slices) {
     for (uint32_t t = tid; t < (uint32_t)(2 * SLICE); t += NT) (&S.t.sl.tab[0][0])[t] = 0u;
   }
-  if (mode == M_TOPK) S.hist[tid] = 0u;   // HB == NT
+  if (mode == M_TOPK || NUC) S.hist[tid] = 0u;   // HB == NT
   lds_barrier();
   uint32_t my_flags = 0;
   if (has_tab && !c.err) {
@@ -5308,6 +5731,91 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
     }
   }
   stamp(A, row, chunk, 4);
+  if (NUC && emit && has_tab) {
+    // a row with penalties or biases also leaves its adjusted logits for a
+    // finisher that has to read the whole row
+#pragma unroll
+    for (int i = 0; i < PER_MAX; ++i) {
+      const uint32_t e0 = c0 + (uint32_t)i * SLICE + tid * 4u;
+      if (i < (int)A.per && e0 < c1) {
+        auto* ap = reinterpret_cast<unsigned long long*>(A.w.adj + (uint64_t)row * ((V + 3u) & ~3u) + e0);
+        st_dev(ap, ((unsigned long long)__float_as_uint(lv[i][1]) << 32) | __float_as_uint(lv[i][0]));
+        st_dev(ap + 1, ((unsigned long long)__float_as_uint(lv[i][3]) << 32) | __float_as_uint(lv[i][2]));
+      }
+    }
+  }
+  // Nucleus candidates.  The legal logits are counted on a 1/32-octave
+  // grid of their weights below the chunk maximum (those 32 octaves down
+  // are left out), each bin's mass bounded by its count times its upper
+  // edge.  The threshold is the bin edge below which the chunk holds at
+  // most (1 - top_p) / (2 C) of its mass and all but NUC_MIN / C of its
+  // tokens, and at least so high that CCAP / C tokens are listed (the
+  // finisher caches CCAP): chunks whose tails are alike then leave at most half the row's
+  // allowance below the largest of their thresholds, and a chunk that
+  // holds one large weight still lists the tokens that rank beside the
+  // other chunks' heads.  The finisher checks that (a row that fails is
+  // finished over the whole row).  A token too far below the largest chunk
+  // maximum published so far is no candidate either (nuc_reach).
+  // A chunk of few legal tokens (grammar masks) packs them first, as a
+  // candidate list; beyond nuc_list of them it counts and thins that list,
+  // one to four entries per thread where the registers hold a few legal
+  // lanes per element.
+  // (A row of up to CCAP legal tokens has them spread over its chunks to
+  // within a half, and is decided best with all of them listed: thinning
+  // 6,000 to 7,400 legal tokens of flat bf16 rows left 90% and cost 4 us.
+  // Such chunks sum no mass; beside chunks that thin their lists it counts
+  // as unknown, which sends the row to finish_nuc.)
+  const uint32_t nuc_list = (uint32_t)CCAP / A.C * 3u / 2u;
+  const bool nuc_pack = NUC && emit && nleg <= 4u * (uint32_t)NT;
+  const bool nuc_x = NUC && emit && !nuc_pack;
+  // The row maximum so far (every chunk publishes its own), waited for where
+  // the threshold needs it.
+  unsigned long long xold = 0ull;
+  if (NUC && emit && nleg > nuc_list && tid == 0)
+    xold = __hip_atomic_fetch_max(A.w.rowx + (uint64_t)row * ROWX_STRIDE, ((unsigned long long)A.epoch << 32) | maxkey,
+                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  auto nuc_row_max = [&]() {
+    if (tid == 0) S.xkey = (uint32_t)(xold >> 32) == A.epoch ? max(maxkey, (uint32_t)xold) : maxkey;
+  };
+  // The edge, from the counts in S.hist (hs: bins per logit); every wave
+  // finds it itself, from the far end: lane j sums the bins
+  // [HB - 16 (j + 1), HB - 16 j).
+  auto nuc_edge = [&](const float hs) -> float {
+    const uint32_t b0 = (uint32_t)HB - 16u * (lane() + 1u);
+    float sm = 0.0f;
+    uint32_t cm = 0u, ctop = 0u;   // counts of the group and of its top bin
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint4 h4 = *reinterpret_cast<const uint4*>(&S.hist[b0 + (uint32_t)q * 4u]);
+      const float w0 = __builtin_amdgcn_exp2f(-0.125f * (float)q);
+      sm += w0 * ((float)h4.x + 0x1.f50766p-1f * (float)h4.y + 0x1.ea4afap-1f * (float)h4.z + 0x1.dfc974p-1f * (float)h4.w);
+      cm += h4.x + h4.y + h4.z + h4.w;
+      if (q == 0) ctop = h4.x;
+    }
+    sm *= __builtin_amdgcn_exp2f((float)b0 * -0.03125f);
+    const double sd = (double)sm, inc = wave_scan_f64(sd);
+    const uint32_t ci = wave_scan_u32(cm), ct = bcast63(ci), cmin = NUC_MIN / A.C, cap = (uint32_t)CCAP / A.C;
+    const double allow = (1.0 - c.top_p) / (double)(2u * A.C) * bcast63(inc);
+    const uint64_t reach = __builtin_amdgcn_ballot_w64((inc > allow || ci + cmin > ct) && ci - ctop + cap >= ct);
+    const uint32_t g = reach ? (uint32_t)__builtin_ctzll(reach) : 63u;
+    const double below = readlane_t(inc - sd, g);
+    const uint32_t cbelow = (uint32_t)__builtin_amdgcn_readlane((int)(ci - cm), (int)g);
+    const uint32_t bin = (uint32_t)HB - 16u * g - 1u - (lane() & 15u);
+    const uint32_t hv = lane() < 16u ? S.hist[bin] : 0u;
+    const double v = (double)((float)hv * __builtin_amdgcn_exp2f((float)bin * -0.03125f));
+    const double vi = below + wave_scan_f64(v);
+    const uint32_t hi = cbelow + wave_scan_u32(hv);
+    const uint64_t r2 = __builtin_amdgcn_ballot_w64(lane() < 16u && (vi > allow || hi + cmin > ct) && hi - hv + cap >= ct);
+    const uint32_t tb = (uint32_t)HB - 16u * g - 1u - (r2 ? (uint32_t)__builtin_ctzll(r2) : 15u);
+    const float drop = (float)(tb + 1u) / hs;
+    const float thr1 = tb >= (uint32_t)HB - 1u ? -INFINITY : m - drop - (fabsf(m) + drop) * 1e-6f;
+    const double lim = (double)okey_value(S.xkey) - nuc_reach;
+    const float thr2 = (float)lim - fabsf((float)lim) * 1e-6f - 1e-30f;
+    const float t = vmax(thr1, thr2);
+    // no such edge (a bin of more than CCAP / C tokens at the top), or a
+    // NaN from an overflowing 1 / T: nothing is listed
+    return !reach || !r2 || !(t < INFINITY) ? INFINITY : t;
+  };
   const bool mass32 = row_ok && nleg > 0 &&
                       ((mode == M_MINP && c.top_p < 1.0) || (mode == M_TOPK && masked_row));
   // (all-candidates rows emit every legal token: the finisher's own f64
@@ -5329,7 +5837,7 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
         const uint32_t sbase = c0 + (uint32_t)i * SLICE;
         const bool full = !masked_row && min(c1, sbase + (uint32_t)SLICE) - sbase == (uint32_t)SLICE;
         const uint32_t qb = full ? 0xfu : (uint32_t)(lq >> (4 * i)) & 0xfu;
-        if (emit && !minp_x) {
+        if (emit && !minp_x && !nuc_x) {
           // screen the slice on the quad maxima (legal tokens only) first
           uint32_t cnt = 0;
           if (__builtin_amdgcn_ballot_w64(qm[i] >= thr)) {
@@ -5401,7 +5909,7 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
             if (lane() == 0) st_dev(&A.w.seg[(((uint64_t)row * MAXC + chunk) * PER_MAX + i) * NW + wave()], ws);
           }
         }
-      } else if (lane() == 0 && emit) {
+      } else if (lane() == 0 && emit && !nuc_x) {
         S.wcnt[i * NW + wave()] = 0u;
       }
     }
@@ -5441,12 +5949,64 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
       }
     }
   }
+  if (nuc_x) {
+    const float c2 = (float)(invT * 1.4426950408889634);
+    const float hs = c2 * 32.0f;
+#pragma unroll
+    for (int i = 0; i < PER_MAX; ++i) {
+      if (i < (int)A.per) {
+        const uint32_t sbase = c0 + (uint32_t)i * SLICE;
+        const bool full = !masked_row && min(c1, sbase + (uint32_t)SLICE) - sbase == (uint32_t)SLICE;
+        const uint32_t qb = full ? 0xfu : (uint32_t)(lq >> (4 * i)) & 0xfu;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float d = (m - lv[i][e]) * hs;
+          if (((qb >> e) & 1u) && d < (float)HB) atomicAdd(&S.hist[(uint32_t)d], 1u);
+        }
+      }
+    }
+    nuc_row_max();
+    lds_barrier();
+    thr = nuc_edge(hs);
+    // counts, and the f32 mass of the tokens below the threshold (they hold
+    // a small share of the row; the candidates' mass is summed in f64 below)
+#pragma unroll
+    for (int i = 0; i < PER_MAX; ++i) {
+      cnt_i[i] = 0u;
+      uint32_t cnt = 0;
+      if (i < (int)A.per) {
+        const uint32_t sbase = c0 + (uint32_t)i * SLICE;
+        const bool full = !masked_row && min(c1, sbase + (uint32_t)SLICE) - sbase == (uint32_t)SLICE;
+        const uint32_t qb = full ? 0xfu : (uint32_t)(lq >> (4 * i)) & 0xfu;
+        if (__builtin_amdgcn_ballot_w64(qm[i] >= thr)) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            cnt += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(((qb >> e) & 1u) && lv[i][e] >= thr));
+        }
+        cnt_i[i] = cnt;
+        float sw = 0.0f, ew = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float y = vmax((lv[i][e] - m) * c2, -200.0f);
+          const float w = ((qb >> e) & 1u) && !(lv[i][e] >= thr) ? __builtin_amdgcn_exp2f(y) : 0.0f;
+          sw += w;
+          ew = __builtin_fmaf(w, -y, ew);
+        }
+        m0 += (double)sw;
+        m1 += (double)ew;
+      }
+      if (lane() == 0) S.wcnt[i * NW + wave()] = cnt;
+    }
+  }
   stamp(A, row, chunk, 5);
   if (emit || mass32 || mass64) lds_barrier();
   if (mass32 || mass64) {
+    // (thread 0 publishes the mass: wave 0 combines the waves' sums)
     double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) { s0 += S.wq[w].m0; s1 += S.wq[w].m1; }
+    if (wave() == 0) {
+      s0 = wave_sum_f64(lane() < (uint32_t)NW ? S.wq[lane()].m0 : 0.0);
+      s1 = mass32 ? wave_sum_f64(lane() < (uint32_t)NW ? S.wq[lane()].m1 : 0.0) : 0.0;
+    }
     mass = s0;
     if (mass32) {
       // |mass - sum of exact weights| <= 1.01 (2^-22 S + 3 2^-24 S) for the
@@ -5472,6 +6032,12 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
     ncand = t0 + t1s + t2s;
     const uint32_t x0 = i0 - v0, x1 = i1 - v1 + t0, x2 = i2 - v2 + t0 + t1s;
     const uint64_t cbase = rbase + c0;
+    // as the lean body: staged in LDS (the count tables are dead by now),
+    // then copied out with coalesced stores
+    const bool staged = ncand <= (uint32_t)(CHUNK_MAX / 4);   // uniform
+    float* stl = reinterpret_cast<float*>(S.t.ct);
+    uint32_t* sti = S.t.ct + CHUNK_MAX / 4;
+    double cpart = 0.0;   // nucleus rows: this thread's share of the candidates' mass
 #pragma unroll
     for (int i = 0; i < PER_MAX; ++i) {
       if (i < (int)A.per && cnt_i[i]) {
@@ -5495,13 +6061,71 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           if (em[e]) {
-            const uint64_t pos = cbase + off;
-            st_dev(&A.w.cand_l[pos], lv[i][e]);
-            st_dev(&A.w.cand_id[pos], e0 + (uint32_t)e);
+            if (staged) {
+              stl[off] = lv[i][e];
+              sti[off] = e0 + (uint32_t)e;
+            } else {
+              const uint64_t pos = cbase + off;
+              st_dev(&A.w.cand_l[pos], lv[i][e]);
+              st_dev(&A.w.cand_id[pos], e0 + (uint32_t)e);
+            }
             ++off;
           }
         }
       }
+    }
+    if (nuc_pack && nleg > nuc_list) {
+      lds_barrier();
+      const float hs = (float)(invT * 1.4426950408889634) * 32.0f;
+      const uint32_t R = (ncand + (uint32_t)NT - 1u) / (uint32_t)NT, j0 = tid * R;
+      float pl[4];
+      uint32_t pi[4], kb = 0u;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const bool in = (uint32_t)r < R && j0 + (uint32_t)r < ncand;
+        pl[r] = in ? stl[j0 + (uint32_t)r] : -INFINITY;
+        pi[r] = in ? sti[j0 + (uint32_t)r] : 0u;
+        const float d = (m - pl[r]) * hs;
+        if (in && d < (float)HB) atomicAdd(&S.hist[(uint32_t)d], 1u);
+        if (in) cpart += exp_neg_t(((double)pl[r] - md) * invT, S.etab, S.etab + 64);
+      }
+      nuc_row_max();
+      lds_barrier();
+      thr = nuc_edge(hs);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) kb |= (uint32_t)r < R && j0 + (uint32_t)r < ncand && pl[r] >= thr ? 1u << r : 0u;
+      uint32_t at = block_excl_scan_u32((uint32_t)__builtin_popcount(kb), S.wcnt, &ncand);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if ((kb >> r) & 1u) { stl[at] = pl[r]; sti[at] = pi[r]; ++at; }
+    }
+    if (staged) {
+      lds_barrier();
+      for (uint32_t j = tid; j < ncand; j += NT) {
+        const float l = stl[j];
+        st_dev(&A.w.cand_l[cbase + j], l);
+        st_dev(&A.w.cand_id[cbase + j], sti[j]);
+        if (nuc_x) cpart += exp_neg_t(((double)l - md) * invT, S.etab, S.etab + 64);
+      }
+    }
+    if (nuc_pack && nleg <= nuc_list) mass_err = INFINITY;   // all listed, not summed
+    if (nuc_x || (nuc_pack && nleg > nuc_list)) {
+      const double w0s = wave_sum_f64(m0), w1s = wave_sum_f64(m1), w2s = wave_sum_f64(cpart);
+      if (lane() == 0) { S.wq[wave()].m0 = w0s; S.wq[wave()].m1 = w1s; S.wp[wave()].m0 = w2s; }
+      lds_barrier();
+      // (thread 0 publishes the mass: wave 0 combines the waves' sums)
+      const bool lw = lane() < (uint32_t)NW;
+      double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+      if (wave() == 0) {
+        s0 = wave_sum_f64(lw ? S.wq[lane()].m0 : 0.0);
+        s1 = wave_sum_f64(lw ? S.wq[lane()].m1 : 0.0);
+        s2 = wave_sum_f64(lw ? S.wp[lane()].m0 : 0.0);
+      }
+      mass = s0 + s2;
+      // the f32 part as above; the f64 part as a wide min-p chunk's
+      mass_err = 1.01 * (0x1p-22 * s0 + 3.0 * 0x1p-24 * s0 + 0.6931471805599453 * 3.0001 * 0x1p-24 * s1) +
+                 (double)nleg * 0x1p-124 + 0x1p-40 * s0 + sum_bound(s2, nleg + (uint32_t)NT, 8.0) +
+                 3.0 * 0.37 * (double)nleg * mxs::U;
     }
   }
 
@@ -5580,7 +6204,8 @@ __global__ __launch_bounds__(NT) void sample_kernel(
         else rxw = chunk_fast<In, M_MINP, false, RX>(A, U, c, row, chunk, c0, c1, 0u, 0u, rx);
       }
     } else {
-      rxw = chunk_general<In>(A, U, c, row, chunk, rx);
+      if (!c.err && nucleus_only(c, V)) rxw = chunk_general<In, true>(A, U, c, row, chunk, rx);
+      else rxw = chunk_general<In, false>(A, U, c, row, chunk, rx);
     }
   }
   // The step receipt's reload paths run here, after the body, where its
@@ -5622,7 +6247,13 @@ __global__ __launch_bounds__(NT) void sample_kernel(
   stamp(A, row, MAXC, 0);
   FinLoads P;
   fin_issue(A, row, P);
-  finish_row<In>(A, U.f, c, row, mode, (uint64_t)row * V, c.greedy ? 0.0 : 1.0 / c.T, P);
+  // (a nucleus row its candidates could not decide is finished over the
+  // whole row)
+  if (finish_row<In>(A, U.f, c, row, mode, (uint64_t)row * V, c.greedy ? 0.0 : 1.0 / c.T, P,
+                     !c.err && nucleus_only(c, V))) {
+    __syncthreads();   // the finisher's LDS is free
+    finish_nuc<In>(A, U.f, c, row, 1.0 / c.T);
+  }
   stamp(A, row, MAXC, 7);
   if (RX && rx) {
     __syncthreads();   // the finisher's LDS is free
@@ -6115,7 +6746,7 @@ __global__ __launch_bounds__(NT) void tile_finish_kernel(SampleArgs A, const Epi
   __syncthreads();
   FinLoads P;
   fin_issue(A, row, P);
-  finish_row<float>(A, U.f, c, row, mode, rbase, c.greedy ? 0.0 : 1.0 / c.T, P);
+  finish_row<float>(A, U.f, c, row, mode, rbase, c.greedy ? 0.0 : 1.0 / c.T, P, false);
 }
 
 }  // namespace mxs
@@ -6247,8 +6878,12 @@ int mxs_create(int device, void* stream, uint32_t max_rows, uint32_t max_vocab, 
   e = e ? e : hipMalloc(&ctx->work.ctr, (size_t)max_rows * mxs::CTR_STRIDE * sizeof(uint32_t));
   e = e ? e : hipMalloc(&ctx->work.rowx, (size_t)max_rows * mxs::ROWX_STRIDE * sizeof(unsigned long long));
   e = e ? e : hipMalloc(&ctx->work.stat, (size_t)max_rows * mxs::MAXC * sizeof(mxs::ChunkStat));
-  e = e ? e : hipMalloc(&ctx->work.cand_l, rv * sizeof(float));
-  e = e ? e : hipMalloc(&ctx->work.cand_id, rv * sizeof(uint32_t));
+  // the candidate lists and the adjusted logits: one allocation, 256-byte steps
+  const size_t list_n = (rv + 63u) & ~(size_t)63u;
+  e = e ? e : hipMalloc(&ctx->work.cand_l,
+                        (2u * list_n + (size_t)max_rows * ((max_vocab + 3u) & ~3u)) * sizeof(float));
+  ctx->work.cand_id = reinterpret_cast<uint32_t*>(ctx->work.cand_l + list_n);
+  ctx->work.adj = ctx->work.cand_l + 2u * list_n;
   e = e ? e : hipMalloc(&ctx->work.seg, (size_t)max_rows * mxs::MAXC * mxs::PER_MAX * mxs::NW * sizeof(double));
   e = e ? e : hipMalloc(&ctx->work.cand_rows, (size_t)max_rows * sizeof(int32_t));
   e = e ? e : hipMemset(ctx->work.cand_rows, 0xff, (size_t)max_rows * sizeof(int32_t));
@@ -6302,8 +6937,7 @@ int mxs_destroy(mxs_ctx* ctx) {
   hipFree(ctx->work.ctr);
   hipFree(ctx->work.rowx);
   hipFree(ctx->work.stat);
-  hipFree(ctx->work.cand_l);
-  hipFree(ctx->work.cand_id);
+  hipFree(ctx->work.cand_l);   // and cand_id, adj
   hipFree(ctx->work.seg);
   hipFree(ctx->work.cand_rows);
   hipFree(ctx->d_zero_u32);

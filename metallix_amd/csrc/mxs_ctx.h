@@ -60,6 +60,7 @@ struct Work {
   ChunkStat* stat;            // [max_rows * MAXC]
   float* cand_l;              // [max_rows * max_vocab]
   uint32_t* cand_id;          // [max_rows * max_vocab]
+  float* adj;                 // [max_rows * roundup4(max_vocab)] adjusted logits of top-p rows with penalties or biases
   double* seg;                // [max_rows * MAXC * PER_MAX * NW]
   int32_t* cand_rows;         // [max_rows] candidates the row's finisher chose from (-1: no list)
 };

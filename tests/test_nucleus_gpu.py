@@ -1,0 +1,152 @@
+"""Top-p rows without a top-k or min-p: chunk candidates with their mass
+certificate, and the whole-row finish behind them, against the oracle
+(nucleus_mask, crates/app/cli/src/qwen_forward.rs:474-549).  Statuses, kept
+sets, adjusted logits and tokens are bit-exact."""
+import numpy as np
+import pytest
+
+from helpers import compare, run_gpu
+
+pytestmark = pytest.mark.gpu
+
+LARGE = 11   # MXS_PATH_LARGE
+
+
+@pytest.fixture(scope="module")
+def torch_mod():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch
+
+
+def text_row(rng, V, fall, spread=2.5):
+    x = (spread * rng.standard_normal(V)).astype(np.float32)
+    n = min(4096, max(1, V // 2))
+    ids = rng.choice(V, n, replace=False)
+    x[ids] = np.maximum(x[ids], 20.0 - fall * np.log(np.arange(1, n + 1))).astype(np.float32)
+    return x
+
+
+def rows_of(kind, rng, R, V):
+    if kind == "text":       # nuclei of a few to thousands of tokens
+        return np.stack([text_row(rng, V, 1.1 + 0.4 * (r % 8)) for r in range(R)])
+    if kind == "flat":       # nuclei of most of the row
+        return (0.5 + 0.5 * (np.arange(R)[:, None] % 4)).astype(np.float32) * rng.standard_normal((R, V)).astype(np.float32)
+    if kind == "steps":      # crowded bins: a few values, each thousands of times
+        v = rng.standard_normal((R, 7)).astype(np.float32)
+        return v[np.arange(R)[:, None], rng.integers(0, 7, (R, V))]
+    if kind == "one_head":   # all head mass in one chunk, the others flat
+        x = rng.standard_normal((R, V)).astype(np.float32)
+        x[:, : max(1, V // 40)] += 9.0
+        return x
+    if kind == "lowest":     # most tokens at the lowest finite value
+        x = np.full((R, V), np.finfo(np.float32).min, dtype=np.float32)
+        n = min(V, 300)
+        for r in range(R):
+            x[r, rng.choice(V, n, replace=False)] = rng.standard_normal(n)
+        return x
+    raise ValueError(kind)
+
+
+def batch(kind, R, V, bf16=False, history=0, bias=0, mask=False, seed=0):
+    from metallix_amd.synth import Batch, bf16_bits_to_f32, to_bf16_bits
+
+    rng = np.random.default_rng([R, V, seed])
+    x = rows_of(kind, rng, R, V)
+    bits = None
+    if bf16:
+        bits = to_bf16_bits(x)
+        x = bf16_bits_to_f32(bits)
+    b = Batch(name=f"nucleus-{kind}", logits=x, temperature=rng.uniform(0.5, 1.5, R), uniform=rng.random(R),
+              top_p=np.array([0.05, 0.5, 0.9, 0.95, 0.99, 0.9999, 1.0 - 1e-9, 0.8])[np.arange(R) % 8], bf16_bits=bits,
+              tokenizer_vocab=V)
+    if history:
+        b.history_offsets = (np.arange(R + 1) * history).astype(np.uint32)
+        b.history_ids = rng.integers(0, V, R * history).astype(np.uint32)
+        b.repetition = np.where(np.arange(R) % 2, 1.2, 0.9).astype(np.float32)
+        b.presence = np.full(R, 0.4, dtype=np.float32)
+        b.frequency = np.full(R, 0.1, dtype=np.float32)
+    if bias:
+        b.bias_offsets = (np.arange(R + 1) * bias).astype(np.uint32)
+        b.bias_ids = np.concatenate([np.sort(rng.choice(V, bias, replace=False)) for _ in range(R)]).astype(np.uint32)
+        vals = rng.uniform(-3, 3, R * bias).astype(np.float32)
+        vals[::5] = -np.inf
+        b.bias_values = vals
+    if mask:
+        words = (V + 31) // 32
+        m = rng.integers(0, 2 ** 32, (R, words), dtype=np.uint64).astype(np.uint32)
+        m[::2] &= rng.integers(0, 2 ** 32, (len(m[::2]), words), dtype=np.uint64).astype(np.uint32)
+        m[:, 0] |= 1
+        b.mask_words = m
+        b.tokenizer_vocab = max(1, V - 5)
+    return b
+
+
+CASES = [
+    # (kind, rows, vocab, options): the chunk and segment edges of the layout
+    ("text", 8, 1, {}), ("text", 8, 5, {}), ("text", 8, 4097, {}), ("text", 8, 40963, {}),
+    ("text", 16, 151936, {}), ("text", 72, 50257, dict(bf16=True)), ("text", 8, 262144, {}),
+    ("text", 8, 100003, dict(history=700)), ("text", 8, 100003, dict(history=300, bias=40)),
+    ("text", 16, 151936, dict(mask=True)), ("text", 8, 70001, dict(bf16=True, mask=True, history=50)),
+    ("flat", 8, 151936, {}), ("flat", 8, 50257, dict(bf16=True)), ("flat", 8, 262144, {}),
+    ("flat", 8, 99999, dict(history=3000, bias=7)), ("flat", 8, 151936, dict(mask=True, bf16=True)),
+    ("one_head", 8, 151936, {}), ("one_head", 8, 65541, dict(bias=3)),
+    ("lowest", 8, 151936, {}), ("lowest", 8, 30011, dict(bias=25)),
+]
+
+
+@pytest.mark.parametrize("kind,R,V,opt", CASES, ids=lambda v: str(v))
+def test_nucleus_rows(torch_mod, orc, kind, R, V, opt):
+    from metallix_amd import Sampler
+
+    b = batch(kind, R, V, **opt)
+    print(f"case nucleus {kind} rows {R} vocab {V} {opt}", flush=True)
+    s = Sampler(max_rows=R, max_vocab=V)
+    gpu = run_gpu(torch_mod, s, b)
+    s.close()
+    # top_p = 1 - 1e-9 cuts among weights near the f64 sums' error bound: only
+    # such a row may report status 1
+    unc = np.nonzero(gpu["status"] == 1)[0]
+    assert (b.top_p[unc] > 0.99999).all(), (unc, b.top_p[unc])
+    compare(b, gpu, orc.sample_batch(b, debug=True), allow_uncertified=len(unc))
+
+
+@pytest.mark.parametrize("V,bf16", [(20000, False), (151936, True)])
+def test_crowded_bins(torch_mod, orc, V, bf16):
+    """Seven values per row, thousands of tokens each: the cut lies among
+    equal keys (cut by their count and ID).  A prefix sum that equals theta
+    to within the bound is the only uncertified case, and these have none."""
+    from metallix_amd import Sampler
+
+    b = batch("steps", 8, V, bf16=bf16, seed=3)
+    s = Sampler(max_rows=8, max_vocab=V)
+    print(f"case nucleus steps vocab {V} bf16 {bf16}", flush=True)
+    gpu = run_gpu(torch_mod, s, b)
+    s.close()
+    compare(b, gpu, orc.sample_batch(b, debug=True))
+
+
+def test_paths(torch_mod, orc):
+    """A peaked batch is decided from its candidates, a flat one over the
+    whole row; results are the same through either (the two above)."""
+    from helpers import to_device
+    from metallix_amd import Sampler
+
+    torch, V = torch_mod, 151936
+    s = Sampler(max_rows=8, max_vocab=V)
+    buf = torch.zeros(8, dtype=torch.int32, device="cuda")
+    s.lib.mxs_debug_set_paths(s.ctx, buf.data_ptr())
+    for kind, large in (("text", False), ("flat", True)):
+        b = batch(kind, 8, V)
+        b.top_p, b.temperature = np.full(8, 0.9), np.full(8, 0.6)
+        if kind == "text":
+            b.logits = np.stack([text_row(np.random.default_rng(r), V, 2.5) for r in range(8)])
+        logits, kw = to_device(torch, b)
+        s.sample(logits, **kw)
+        torch.cuda.synchronize()
+        got = buf.cpu().numpy()
+        assert ((got == LARGE) == large).all(), (kind, got)
+    s.lib.mxs_debug_set_paths(s.ctx, None)
+    s.close()
