@@ -23,8 +23,8 @@
 // (about 2^-50 (1 + |g| + |score|) each); otherwise the row's status is 1
 // (uncertified) and it carries the device's winner.
 //
-// Launch: grid (8 C, rows / 8) of RNT-thread workgroups; chunk c of a row covers
-// tokens [c RT, (c + 1) RT), 32 tokens RNT apart per thread.
+// Launch: rows * C workgroups of RNT threads; chunk c of a row covers tokens
+// [c RT, (c + 1) RT), RPT / 2 token pairs 2 RNT tokens apart per thread.
 // Each chunk reduces its kept tokens to a RaceStat; the row's last chunk to
 // arrive (device-scope counter) merges them and writes the row's result.
 #include <hip/hip_runtime.h>
@@ -38,7 +38,9 @@ namespace mxs {
 
 constexpr int RNT = 256;                       // threads per race workgroup
 constexpr int RNW = RNT / 64;
-constexpr uint32_t RT = (uint32_t)RNT * 32u;    // tokens per race chunk
+constexpr uint32_t RPT = 16;                    // tokens per thread
+constexpr uint32_t RT = (uint32_t)RNT * RPT;    // tokens per race chunk
+constexpr uint32_t RKW = RT / 32u;              // kept-set words per chunk
 
 // One chunk's kept tokens, reduced.
 struct alignas(16) RaceStat {
@@ -83,6 +85,14 @@ struct RaceArgs {
   RaceStat* stat;           // rows x C
 };
 
+// The 64-bit product of two 32-bit words in one instruction (the compiler
+// takes a high and a low multiply, each at a quarter of the rate).
+__device__ __forceinline__ uint64_t mul_u64(uint32_t a, uint32_t b) {
+  uint64_t d, carry;
+  __asm__("v_mad_u64_u32 %0, %1, %2, %3, 0" : "=v"(d), "=s"(carry) : "s"(a), "v"(b));
+  return d;
+}
+
 // Philox4x32 with 10 rounds (Salmon et al., SC'11; race.rs:39-54).
 __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32_t k1) {
 #pragma unroll
@@ -91,13 +101,12 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32
       k0 += 0x9E3779B9u;
       k1 += 0xBB67AE85u;
     }
-    const uint32_t hi0 = __umulhi(0xD2511F53u, c[0]), lo0 = 0xD2511F53u * c[0];
-    const uint32_t hi1 = __umulhi(0xCD9E8D57u, c[2]), lo1 = 0xCD9E8D57u * c[2];
-    const uint32_t n0 = hi1 ^ c[1] ^ k0, n2 = hi0 ^ c[3] ^ k1;
+    const uint64_t p0 = mul_u64(0xD2511F53u, c[0]), p1 = mul_u64(0xCD9E8D57u, c[2]);
+    const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c[1] ^ k0, n2 = (uint32_t)(p0 >> 32) ^ c[3] ^ k1;
     c[0] = n0;
-    c[1] = lo1;
+    c[1] = (uint32_t)p1;
     c[2] = n2;
-    c[3] = lo0;
+    c[3] = (uint32_t)p0;
   }
 }
 
@@ -121,28 +130,26 @@ __device__ __forceinline__ double gumbel_from_bits(uint64_t bits) {
   return -log(e);
 }
 
-// The same noise in f32, for screening: E from the bits' f32 image (relative
-// error about 2^-22 either branch; the w branch keeps log1p's precision for
-// small w), then f32 logs (about 2 ulp each).  |g32 - g| < 1e-5.
-__device__ __forceinline__ float gumbel32(uint64_t bits) {
-  const uint32_t hi = (uint32_t)(bits >> 32), lo = (uint32_t)bits;
-  float e;
-  if (!(hi >> 31)) {
-    const float w = ((float)hi + ((float)lo + 0.5f) * 0x1p-32f) * 0x1p-32f;
-    e = -log1pf(-w);
-  } else {
-    const float v = ((float)(~hi) + ((float)(~lo) + 0.5f) * 0x1p-32f) * 0x1p-32f;
-    e = -logf(v);
-  }
-  return -logf(e);
+// The same noise in f32, for screening: g = -ln e, e = -ln v, v = 1 - w the
+// complement of the noise variate w, on the hardware log2 (about an ulp).
+// Below w = 2^-10, e = w + w^2 / 2 (relative error under 2^-21); above it
+// v's f32 rounding (2^-24 absolute) costs e at most 2^-14 relative.  So
+// |g32 - g| < 2^-13.  (The library's log1pf and logf, evaluated on both
+// sides of a divergent branch, took about 75 instructions per token.)
+__device__ __forceinline__ float gumbel32(uint32_t hi, uint32_t lo) {
+  const float w = ((float)hi + (float)lo * 0x1p-32f + 0x1p-33f) * 0x1p-32f;
+  const float v = ((float)(~hi) + (float)(~lo) * 0x1p-32f + 0x1p-33f) * 0x1p-32f;
+  const float big = __builtin_amdgcn_logf(v) * -0.69314718f;
+  const float e = w < 0x1p-10f ? __builtin_fmaf(0.5f * w, w, w) : big;
+  return __builtin_amdgcn_logf(e) * -0.69314718f;
 }
 
 // Bound on |s32 - (l / T + g - m / T)| for the f32 screening score
 // s32 = (l - m) * (1/T)_f32 + g32 (m the row's largest adjusted logit, at or
 // above every kept logit):
 // (l - m) / T <= 0 and g <= 45.1 give |(l - m) / T| <= |s32| + 46, whose
-// three f32 roundings cost under 2^-22.4 (|s32| + 46); plus |g32 - g| and
-// the final rounding.  The form below is several times larger than that.
+// three f32 roundings cost under 2^-22.4 (|s32| + 46); plus |g32 - g| < 2^-13
+// and the final rounding.  The form below is several times larger than that.
 __device__ __forceinline__ float err32(float s32) { return 0x1p-10f + fabsf(s32) * 0x1p-19f; }
 
 // Certification margin between the two best device scores.
@@ -183,6 +190,52 @@ __device__ __forceinline__ void cnt_add_sat(uint32_t* p, uint32_t sh) {
   }
 }
 
+// exp_neg_p (mxs_math.h: the same operations and results) with the
+// polynomial's coefficients held in scalar registers across the token loop:
+// as literals each took two moves per use, twice the polynomial itself.
+struct ExpCoef {
+  double c[12];   // 1/13! .. 1/2!
+  __device__ __forceinline__ void load() {
+    const double v[12] = {1.0 / 6227020800.0, 1.0 / 479001600.0, 1.0 / 39916800.0, 1.0 / 3628800.0, 1.0 / 362880.0,
+                          1.0 / 40320.0, 1.0 / 5040.0, 1.0 / 720.0, 1.0 / 120.0, 1.0 / 24.0, 1.0 / 6.0, 0.5};
+#pragma unroll
+    for (int i = 0; i < 12; ++i) {
+      c[i] = v[i];
+      __asm__ volatile("" : "+s"(c[i]));
+    }
+  }
+  __device__ __forceinline__ double operator()(double x) const {
+    const double t = rint(x * 1.4426950408889634);
+    double r = fma(-t, 0.6931471803691238, x);
+    r = fma(-t, 1.9082149292705877e-10, r);
+    double p = c[0];
+#pragma unroll
+    for (int i = 1; i < 12; ++i) p = fma(p, r, c[i]);
+    p = fma(p, r, 1.0);
+    const double e = ldexp(fma(p, r, 1.0), (int)t);
+    return x > -746.0 ? e : 0.0;
+  }
+};
+
+// Two consecutive logits (the first token ID even, in range: the row stride
+// is a multiple of 4, so the second is inside the row's stride).
+template <typename In>
+struct Pair;
+template <>
+struct Pair<float> {
+  __device__ static void load(const float* p, float x[2]) {
+    const float2 v = *reinterpret_cast<const float2*>(p);
+    x[0] = v.x; x[1] = v.y;
+  }
+};
+template <>
+struct Pair<uint16_t> {
+  __device__ static void load(const uint16_t* p, float x[2]) {
+    const uint32_t v = *reinterpret_cast<const uint32_t*>(p);
+    x[0] = bf16_to_f32((uint16_t)(v & 0xffffu)); x[1] = bf16_to_f32((uint16_t)(v >> 16));
+  }
+};
+
 struct RaceSmem {
   uint32_t cnt[RT / 2];      // history counts of the chunk's tokens (16-bit pairs)
   float redf2[RNW];
@@ -190,24 +243,27 @@ struct RaceSmem {
   double b1[RNW], b2[RNW];
   uint32_t bid[RNW];
   float bl[RNW];
-  uint32_t kw[RNT];          // the chunk's kept-set words
+  uint32_t kw[RKW];          // the chunk's kept-set words
   uint32_t any, last;
 };
 
 template <typename In>
 __global__ __launch_bounds__(RNT) void race_kernel(RaceArgs A) {
   __shared__ RaceSmem S;
-  // blockIdx.x = chunk * 8 + xcd and row = blockIdx.y * 8 + xcd: workgroup
-  // i runs on XCD i mod 8, so a row's chunks share one XCD's L2.
-  const uint32_t tid = threadIdx.x, chunk = blockIdx.x >> 3, row = blockIdx.y * 8u + (blockIdx.x & 7u);
-  if (row >= A.rows) return;
+  // Workgroups in (row, chunk) order: workgroup i runs on XCD i mod 8, so a
+  // row's chunks spread over the XCDs.  A whole-row race is compute (about
+  // 450 cycles per 64 tokens), its chunks share only the kept words and the
+  // history, and one XCD per row left the others idle when the heavy rows
+  // fell on few of them (half the rows whole-row races, every second row:
+  // race_kernel 85 us, four XCDs busy).
+  const uint32_t tid = threadIdx.x, row = blockIdx.x / A.C, chunk = blockIdx.x - row * A.C;
   // Every per-row load goes out at once (the kept words and the row's
   // parameters are in bounds for every row below A.rows).
   const int32_t st0 = A.status[row];
   const double T = A.temperature[row];
   const uint32_t base = chunk * RT;
-  const uint32_t w = chunk * (uint32_t)RNT + tid;
-  uint32_t word = w < A.nwords ? A.kept[(uint64_t)row * A.nwords + w] : 0u;
+  const uint32_t w = chunk * RKW + tid;
+  uint32_t word = tid < RKW && w < A.nwords ? A.kept[(uint64_t)row * A.nwords + w] : 0u;
   const uint32_t hb = A.hoff[row], he = A.hoff[row + 1];
   const uint32_t bb = A.boff[row], be = A.boff[row + 1];
   const float rep = A.rep[row], pres = A.pres[row], freq = A.freq[row];
@@ -215,7 +271,7 @@ __global__ __launch_bounds__(RNT) void race_kernel(RaceArgs A) {
   // Rows the finisher rejected and greedy rows keep the finisher's result.
   if (st0 < 0 || T == 0.0) return;
   if (tid == 0) S.any = 0u;
-  S.kw[tid] = word;
+  if (tid < RKW) S.kw[tid] = word;
   __syncthreads();
   if (word) S.any = 1u;
   __syncthreads();
@@ -230,22 +286,25 @@ __global__ __launch_bounds__(RNT) void race_kernel(RaceArgs A) {
     if (he > hb) {
       for (uint32_t i = tid; i < RT / 2u; i += RNT) S.cnt[i] = 0u;
       __syncthreads();
-      for (uint32_t h = hb + tid; h < he; h += RNT) {
-        const uint32_t d = A.hids[h] - base;
-        if (d < RT) {
-          if (!longh) atomicAdd(&S.cnt[d >> 1], 1u << ((d & 1u) * 16u));
-          else cnt_add_sat(&S.cnt[d >> 1], (d & 1u) * 16u);
-        }
+      for (uint32_t h = hb + tid; h < he; h += 8u * RNT) {   // eight IDs in flight
+        uint32_t d[8];
+#pragma unroll
+        for (uint32_t i = 0; i < 8u; ++i) d[i] = A.hids[min(h + i * RNT, he - 1u)] - base;
+#pragma unroll
+        for (uint32_t i = 0; i < 8u; ++i)
+          if (d[i] < RT && h + i * RNT < he) {
+            if (!longh) atomicAdd(&S.cnt[d[i] >> 1], 1u << ((d[i] & 1u) * 16u));
+            else cnt_add_sat(&S.cnt[d[i] >> 1], (d[i] & 1u) * 16u);
+          }
       }
       __syncthreads();
     }
     const In* lrow = reinterpret_cast<const In*>(A.logits) + (uint64_t)row * A.stride;
-    // The adjusted logit of a kept token (the chunk pass's bias and penalty
-    // stage, penalize_logit).
-    auto adjusted = [&](uint32_t id) -> float {
-      const float l = Quad<In>::one(lrow + id);
+    // The adjusted logit of a kept token with logit l (the chunk pass's bias
+    // and penalty stage, penalize_logit).
+    auto adjust = [&](uint32_t id, float l) -> float {
       uint32_t cnt = 0u;
-      if (he > hb) {
+      if (he > hb) {   // (a pair's second token past the vocabulary has count 0)
         const uint32_t d = id - base;
         cnt = (S.cnt[d >> 1] >> ((d & 1u) * 16u)) & 0xFFFFu;
         if (cnt == 0xFFFFu) {   // saturated (histories above 65535 entries): recount
@@ -261,12 +320,16 @@ __global__ __launch_bounds__(RNT) void race_kernel(RaceArgs A) {
       const bool hasb = lo < be && A.bids[lo] == id;
       return penalize_logit(l, cnt, hasb, hasb ? A.bvals[lo] : 0.0f, rep, pres, freq);
     };
-    // Thread tid takes the chunk's tokens tid + 256 j (j < 32): a wave's
-    // logit loads are consecutive tokens.  Bit j of `mine` is token
-    // tid + 256 j's kept bit (word tid / 32 + 8 j, bit tid mod 32).
+    // Thread tid takes the chunk's token pairs tid + RNT j (j < 8): the two
+    // tokens of a pair share one Philox block (race.rs:66-80), and a wave's
+    // loads are 128 consecutive tokens.  Bits 2 j and 2 j + 1 of `mine` are
+    // pair tid + RNT j's kept bits.
     uint32_t mine = 0u;
-    for (uint32_t j = 0; j < 32u; ++j) mine |= ((S.kw[(tid >> 5) + 8u * j] >> (tid & 31u)) & 1u) << j;
-    const uint32_t id0 = base + tid;
+#pragma unroll
+    for (uint32_t j = 0; j < RPT / 2u; ++j) mine |= ((S.kw[(tid >> 4) + (RNT / 16u) * j] >> (2u * (tid & 15u))) & 3u) << (2u * j);
+    const uint32_t id0 = base + 2u * tid;   // the token of bit b: id0 + 2 RNT (b / 2) + b mod 2
+    // no history (its table is not cleared then) and no bias: the logits as they are
+    const bool plain = he == hb && be == bb;
     // The reference point of the scores and the mass: the row's largest
     // adjusted logit, which the finisher found (the kept set holds it), so
     // no pass over the chunk's tokens precedes the scoring.
@@ -281,16 +344,43 @@ __global__ __launch_bounds__(RNT) void race_kernel(RaceArgs A) {
     float t1 = -INFINITY, t2 = -INFINITY, l1 = 0.0f;
     uint32_t id1 = 0u;
     uint64_t bits1 = 0ull;
-    for (uint32_t r = mine; r; r &= r - 1u) {
-      const uint32_t id = id0 + 256u * (uint32_t)__builtin_ctz(r);
-      const float l = adjusted(id);
-      mass += exp(((double)l - (double)m) * invT);   // (within an ulp of the quotient: the mass feeds only the logprob)
-      const uint64_t bits = race_bits(seed, choice, position, id);
-      const float s32 = (l - m) * invT32 + gumbel32(bits);
-      if (s32 > t1) {
-        t2 = t1; t1 = s32; id1 = id; l1 = l; bits1 = bits;
-      } else {
-        t2 = fmaxf(t2, s32);
+    ExpCoef expo;
+    expo.load();
+    // four pairs' logits in flight per thread
+#pragma unroll
+    for (uint32_t q = 0; q < RPT / 8u; ++q) {
+      const uint32_t mq = (mine >> (8u * q)) & 0xffu;
+      if (!__builtin_amdgcn_ballot_w64(mq != 0u)) continue;
+      float pl[4][2];
+#pragma unroll
+      for (uint32_t j = 0; j < 4u; ++j) {
+        const bool in = ((mq >> (2u * j)) & 3u) != 0u;
+        Pair<In>::load(lrow + (in ? id0 + 2u * RNT * (4u * q + j) : 0u), pl[j]);
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < 4u; ++j) {
+        const uint32_t kb = (mq >> (2u * j)) & 3u;
+        if (!kb) continue;
+        const uint32_t id = id0 + 2u * RNT * (4u * q + j);
+        // (one LDS word holds the pair's history counts)
+        if (!plain && (be > bb || he == hb || S.cnt[(id - base) >> 1] != 0u)) {
+          pl[j][0] = adjust(id, pl[j][0]);
+          pl[j][1] = adjust(id + 1u, pl[j][1]);
+        }
+        uint32_t c4[4] = {id >> 1, position, choice, 0x72616365u};
+        philox4x32_10(c4, (uint32_t)seed, (uint32_t)(seed >> 32));
+#pragma unroll
+        for (uint32_t e = 0; e < 2u; ++e) {
+          if (!((kb >> e) & 1u)) continue;
+          const float l = pl[j][e];
+          mass += expo(((double)l - (double)m) * invT);   // (within ulps of the quotient: the mass feeds only the logprob)
+          const float s32 = (l - m) * invT32 + gumbel32(c4[2u * e], c4[2u * e + 1u]);
+          if (s32 > t1) {
+            t2 = t1; t1 = s32; id1 = id + e; l1 = l; bits1 = ((uint64_t)c4[2u * e] << 32) | c4[2u * e + 1u];
+          } else {
+            t2 = fmaxf(t2, s32);
+          }
+        }
       }
     }
     float smax = t1;
@@ -328,11 +418,11 @@ __global__ __launch_bounds__(RNT) void race_kernel(RaceArgs A) {
       }
     } else
     for (uint32_t r = mine; r; r &= r - 1u) {
-      const uint32_t id = id0 + 256u * (uint32_t)__builtin_ctz(r);
-      const float l = adjusted(id);
+      const uint32_t bt = (uint32_t)__builtin_ctz(r), id = id0 + 2u * RNT * (bt >> 1) + (bt & 1u);
+      const float l = adjust(id, Quad<In>::one(lrow + id));
       const uint64_t bits = race_bits(seed, choice, position, id);
       if (screen) {
-        const float s32 = (l - m) * invT32 + gumbel32(bits);
+        const float s32 = (l - m) * invT32 + gumbel32((uint32_t)(bits >> 32), (uint32_t)bits);
         if (!(s32 + err32(s32) >= cut)) { ++out; continue; }
       }
       const double s = (double)l / T + gumbel_from_bits(bits);
@@ -481,7 +571,7 @@ extern "C" int mxs_sample_race(mxs_ctx* ctx, const mxs_batch* b, const mxs_race*
   int prev = 0;
   (void)hipGetDevice(&prev);
   if (prev != ctx->device) (void)hipSetDevice(ctx->device);
-  const dim3 grid(8u * A.C, (b->rows + 7u) / 8u);
+  const dim3 grid(A.C * b->rows);   // (row, chunk) order
   if (b->dtype == MXS_F32)
     hipLaunchKernelGGL(mxs::race_kernel<float>, grid, dim3(mxs::RNT), 0, ctx->stream, A);
   else
