@@ -8,21 +8,32 @@
 // f64(l) - maximum - log_normalizer.  The caller over-selects top + 8 and
 // filters unspellable IDs, as the reference does.
 //
-// Two launches.  The chunk pass: each row is split into C chunks of TCH tokens, one 256-thread
-// workgroup per chunk (small register and LDS footprints, so several
-// workgroups share a CU and their streams overlap).  A chunk streams its
-// logits once and reduces its maximum and the f64 sum of exp(l - chunk
-// maximum) over weights each within 2^-22 of exact (a corrected f32 exp2;
-// the returned log probabilities stay within 2^-22 relative, see below).  For its top n it takes a threshold that at least n of its
-// tokens reach: each wave's n-th largest lane maximum (n lanes each hold a
-// token at least that large), the largest over the waves.  The tokens at or
-// above it (about n to 2n of 8192 on ordinary rows) are ranked exactly by
-// counting, in (total_cmp descending, ID ascending) order.  A chunk whose
-// threshold admits more than TWCAP tokens in one wave (near-ties) takes an
-// exact radix select instead.  The merge, one workgroup per row, merges the C sorted lists (the entries at or above the largest last
-// entry of a full list, ranked by counting) and the C (maximum, sum) pairs;
-// the launch boundary orders the chunk pass's stores before the merge's
+// Two launches.  The chunk pass: each row is split into C chunks of TCH
+// tokens, one 256-thread workgroup per chunk (small register and LDS
+// footprints, so several workgroups share a CU and their streams overlap).  A
+// chunk streams its logits once and reduces its maximum and the f64 sum of
+// exp(l - chunk maximum) over weights each within 2^-22 of exact (a corrected
+// f32 exp2; the returned log probabilities stay within 2^-22 relative, see
+// below).  For its top n it takes a threshold that at least n of its tokens
+// reach: the smallest over the waves of a wave's ceil(n/4)-th largest lane
+// maximum (so many lanes each hold a token at least that large), rounded
+// down.  The tokens at or above it (about n to 2n of 8192 on ordinary rows)
+// are ranked exactly by counting, in (total_cmp descending, ID ascending)
+// order.  A chunk whose threshold admits more than TWCAP tokens in one wave
+// (near-ties) takes an exact radix select instead.  The merge, one workgroup
+// per row, merges the C sorted lists (the entries at or above the largest
+// last entry of a full list, ranked by counting) and the C (maximum, sum)
+// pairs; the launch boundary orders the chunk pass's stores before the merge's
 // loads, so the chunk workgroups exit without waiting on an arrival counter.
+//
+// Measured (chunk pass and merge, per call, before the unshifted weights, the
+// shared threshold and the merge's early loads -> after): 256 x 262144 f32,
+// n 28, 93.7 -> 68.9 us (268.5 MB at 2.9 -> 3.9 TB/s); 256 x 151936 bf16, n 28,
+// 60.2 -> 44.5 us; 16 x 262144 f32, n 64, 83.5 -> 24.5 us; one row of 151936,
+// n 13, 18.0 -> 15.9 us.  Of the first, weights and merge took 8 us, a shorter
+// threshold search 3 us and the shared threshold 13 us.  Error of the log
+// probabilities against 64 bits, rms over 40 batches of 24 rows: 9.6e-11 ->
+// 7.4e-11.
 
 #include <hip/hip_runtime.h>
 
@@ -91,7 +102,6 @@ struct alignas(16) TopnSmem {
   double etab[128];                                  // 2^(j/64) and its low parts (exp_neg_t)
   uint32_t supw[TCH / 32];                           // the chunk's suppressed tokens (one bit each)
   uint32_t wcnt[TQ * TNW];
-  uint32_t wkept[TNW];
   uint32_t red_u[3][TNW];
   float red_f[TNW];
   double red_d[TNW];
@@ -100,6 +110,16 @@ struct alignas(16) TopnSmem {
 
 __device__ __forceinline__ unsigned long long entry_key(uint32_t k, uint32_t id) {
   return ((unsigned long long)k << 32) | (unsigned long long)(~id);
+}
+
+// exp(x) = w + w r to within the f32 exp2's own error (2^-23) for -86 <= x <=
+// 80: w the exp2 of fl(x log2(e)), r the residual x - fl(x log2(e)) ln 2.
+// 0 from -200 down.
+__device__ __forceinline__ float exp_f32r(float x, float* r) {
+  x = fmaxf(x, -200.0f);
+  const float yh = x * 1.44269504f;
+  *r = __builtin_fmaf(yh, 1.90465421e-9f, __builtin_fmaf(-yh, 0.693147182f, x));   // ln 2 in two parts
+  return __builtin_amdgcn_exp2f(yh);
 }
 
 template <typename In>
@@ -271,29 +291,55 @@ __global__ __launch_bounds__(TNT, 6) void topn_kernel(TopnArgs A) {
   }
   const uint32_t n = A.n;
   const uint32_t take = min(n, len);
-  // This wave's take-th largest lane maximum: `take` lanes hold a token at
-  // least that large, so the chunk's take-th largest token is too (0 when
-  // fewer than `take` lanes hold a token: every token qualifies then).
+  // A threshold that `take` of the chunk's lanes reach, so its take-th largest
+  // token does too: each wave's sh-th largest lane maximum, sh the wave's
+  // share of `take`, and the smallest over the waves (0 where fewer than sh
+  // of a wave's lanes hold a token: every token qualifies then; only a chunk
+  // of less than one slice has such waves).  A wave that answers for all of
+  // `take` alone sets a far lower one: with n 64 its smallest lane maximum,
+  // which an eighth of the tokens pass and overflow the wave's slots.  The
+  // key is rounded down to its upper 18 bits (sign, exponent, 9 mantissa
+  // bits): the other 14 steps of the search are a chain of ballots that would
+  // only spare a few candidates, and the ranking is exact whatever the
+  // threshold.
+  const uint32_t sh = (take + (uint32_t)TNW - 1u) / (uint32_t)TNW;
   const uint64_t actl = __builtin_amdgcn_ballot_w64(t1 > -INFINITY);
   const uint32_t lk = okey(t1);
   uint32_t wthr = 0u;
-  if (take > 0u && (uint32_t)__builtin_popcountll(actl) >= take) {
-    for (int bit = 31; bit >= 0; --bit) {
+  if (take > 0u && (uint32_t)__builtin_popcountll(actl) >= sh) {
+    const uint32_t ak = t1 > -INFINITY ? lk : 0u;
+#pragma unroll
+    for (int bit = 31; bit >= 14; --bit) {
       const uint32_t cand = wthr | (1u << bit);
-      const uint64_t ge = __builtin_amdgcn_ballot_w64(t1 > -INFINITY && lk >= cand);
-      if ((uint32_t)__builtin_popcountll(ge) >= take) wthr = cand;
+      if ((uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(ak >= cand)) >= sh) wthr = cand;
     }
   }
-  // The wave's tokens at or above its threshold go to its LDS region (the
-  // block threshold, the largest of the waves', is applied when ranking);
-  // then the f64 sum of exp(l - t1) relative to this thread's maximum.
+  {
+    const uint32_t kmax = wave_max_u32(lk);
+    const uint64_t anynf = __builtin_amdgcn_ballot_w64(nf);
+    if (lane() == 0) {
+      S.red_u[0][wave()] = kmax;
+      S.red_u[1][wave()] = anynf ? 1u : 0u;
+      S.red_u[2][wave()] = wthr;
+    }
+  }
+  lds_barrier();   // (the exp tables too)
+  uint32_t kmax = 0u, flags = 0u, thr = 0xffffffffu;
+#pragma unroll
+  for (int w = 0; w < TNW; ++w) {
+    kmax = max(kmax, S.red_u[0][w]);
+    flags |= S.red_u[1][w];
+    thr = min(thr, S.red_u[2][w]);
+  }
+  const float m = okey_value(kmax);
+  // The wave's tokens at or above the threshold go to its LDS region; then
+  // the f64 sum of exp(l - t1) relative to this thread's maximum.
   uint32_t woff = 0u;   // this wave's candidates (uniform)
   double part = 0.0;
   if (take > 0u) {
     unsigned long long* wc = S.u.cand + wave() * TWCAP;
-    // (a float compare: a superset of key >= wthr, never an out-of-range
-    // -inf; the ranking filters by key)
-    const float fthr = okey_value(max(wthr, okey(-INFINITY) + 1u));
+    // (a float compare: a superset of key >= thr, never an out-of-range -inf)
+    const float fthr = okey_value(max(thr, okey(-INFINITY) + 1u));
 #pragma unroll
     for (int q = 0; q < TQ; ++q) {
 #pragma unroll
@@ -308,17 +354,54 @@ __global__ __launch_bounds__(TNT, 6) void topn_kernel(TopnArgs A) {
       }
     }
   }
-  lds_barrier();   // the exp tables
-  if (t1 > -INFINITY) {
-    // Each weight 2^y, y = (l - t1) log2(e) <= 0, from the f32 exp2 of y's
-    // f32 head corrected by its tail (y - head, below 2^-24 |y|): within
-    // 2^-22 of exp(l - t1), with no error on the thread maximum's weight 1;
-    // summed in f64.  Every weight but the row maximum's carries at most
-    // that relative error, so the sum S is within 2^-22 (S - 1) and
-    // ln S within 2^-22 (S - 1) / S <= 2^-22 of the exact values, and a
-    // log probability (l - M) - ln S, of magnitude at least (S - 1) / S,
-    // within 2^-22 relative.  y is clamped at -1000 (2^-1000 is 0 in f32):
-    // out-of-range tokens (-inf) and suppressed ones (f32::MIN) weigh 0.
+  // Each weight is an f32 exp2 corrected by the f32 rounding of its argument:
+  // within 2^-22 of exact, with no error on the thread maximum's weight 1;
+  // summed in f64.  Every weight but the row maximum's carries at most that
+  // relative error, so the sum S is within 2^-22 (S - 1) and ln S within
+  // 2^-22 (S - 1) / S <= 2^-22 of the exact values, and a log probability
+  // (l - M) - ln S, of magnitude at least (S - 1) / S, within 2^-22 relative.
+  //
+  // The pass over the chunk is bound by vector instructions, and the f64
+  // difference, scaling and conversions were most of a weight.  A wave whose
+  // logits allow it takes exp(l) itself, unshifted: the residual l - yh ln 2
+  // of yh = fl(l log2(e)) comes from two f32 fmas (the first exact up to one
+  // rounding of a value 2^-24 as large).  It may where no lane's maximum passes
+  // 80 (e^80 in f32 range) and no weight falls below f32's normal range that
+  // would not relative to the lane maximum too: a maximum >= 0, or a minimum
+  // above -86.  The weights are summed in f64, the corrections w r (2^-24 as
+  // large) in f32, which rounds 2^-48 of the lane's sum away; the maximum's
+  // own weight is then taken out of the sum again (the same instructions give
+  // the same bits) and enters as exactly 1.  A wave with a lane whose other
+  // tokens together weigh less than 2^-20 of its maximum, where 2^-48 of the
+  // maximum would show, takes the f64 differences.  Logits below -200
+  // (out-of-range and suppressed tokens too) weigh 0.
+  bool direct = __builtin_amdgcn_ballot_w64(t1 > -INFINITY && !(t1 >= 0.0f && t1 <= 80.0f)) == 0ull;
+  if (!direct) {
+    float tmin = INFINITY;
+#pragma unroll
+    for (int q = 0; q < TQ; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tmin = fminf(tmin, x[q][e]);
+    direct = __builtin_amdgcn_ballot_w64(t1 > -INFINITY && !(t1 <= 80.0f && (t1 >= 0.0f || tmin >= -86.0f))) == 0ull;
+  }
+  if (direct) {
+    float corr = 0.0f, r;
+#pragma unroll
+    for (int q = 0; q < TQ; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float w = exp_f32r(x[q][e], &r);
+        part += (double)w;
+        corr = __builtin_fmaf(w, r, corr);
+      }
+    const float w1 = exp_f32r(t1, &r);
+    part = (part - (double)w1) + ((double)corr - (double)w1 * (double)r);   // the lane's tokens but its maximum
+    direct = __builtin_amdgcn_ballot_w64(t1 > -INFINITY && !(part >= (double)w1 * 0x1p-20)) == 0ull;
+    if (!direct) part = 0.0;
+  }
+  if (!direct && t1 > -INFINITY) {
+    // 2^y, y = (l - t1) log2(e) <= 0 formed in f64 and split into an f32 head
+    // and tail.  y is clamped at -1000 (2^-1000 is 0 in f32).
     const double tm = (double)t1;
 #pragma unroll
     for (int q = 0; q < TQ; ++q)
@@ -331,65 +414,36 @@ __global__ __launch_bounds__(TNT, 6) void topn_kernel(TopnArgs A) {
         part += (double)__builtin_fmaf(eh, yl * 0.69314718f, eh);
       }
   }
-  {
-    const uint32_t kmax = wave_max_u32(lk);
-    const uint64_t anynf = __builtin_amdgcn_ballot_w64(nf);
-    if (lane() == 0) {
-      S.red_u[0][wave()] = kmax;
-      S.red_u[1][wave()] = anynf ? 1u : 0u;
-      S.red_u[2][wave()] = wthr;
-      S.wcnt[wave()] = woff;
+  if (t1 > -INFINITY) {   // the thread's sum rescaled to the chunk maximum
+    const double own = exp_neg_t((double)t1 - (double)m, S.etab, S.etab + 64);
+    if (direct) {
+      const double em = exp_neg_t(-fabs((double)m), S.etab, S.etab + 64);   // m >= t1 >= -86
+      part = own + part * (m >= 0.0f ? em : 1.0 / em);
+    } else {
+      part *= own;
     }
   }
-  lds_barrier();
-  uint32_t kmax = 0u, flags = 0u, lthr = 0u, ncand = 0u, over = 0u;
-  uint32_t wb[TNW];
-#pragma unroll
-  for (int w = 0; w < TNW; ++w) {
-    kmax = max(kmax, S.red_u[0][w]);
-    flags |= S.red_u[1][w];
-    lthr = max(lthr, S.red_u[2][w]);
-    wb[w] = ncand;
-    ncand += S.wcnt[w];
-    over |= S.wcnt[w] > TWCAP ? 1u : 0u;
+  part = wave_sum_f64(part);
+  if (lane() == 0) {
+    S.red_d[wave()] = part;
+    S.wcnt[wave()] = woff;
   }
-  const float m = okey_value(kmax);
+  lds_barrier();
   double sum = 0.0;
   uint32_t listed = 0;
   if (!flags && len > 0) {
-    // the thread's sum rescaled to the chunk maximum
-    if (t1 > -INFINITY) part *= exp_neg_t((double)t1 - (double)m, S.etab, S.etab + 64);
-    part = wave_sum_f64(part);
-    if (lane() == 0) S.red_d[wave()] = part;
+    uint32_t over = 0u;
+#pragma unroll
+    for (int w = 0; w < TNW; ++w) {
+      sum += S.red_d[w];
+      over |= S.wcnt[w] > TWCAP ? 1u : 0u;
+    }
     if (take > 0u && !over) {
-      // ---- the candidates at or above the block threshold: each wave
-      // compacts its own region in place, then they are ranked by counting
-      // (keys are distinct).
-      {
-        const uint32_t wn = S.wcnt[wave()];
-        unsigned long long* wc = S.u.cand + wave() * TWCAP;
-        unsigned long long ev[TWCAP / 64];
-        bool keep[TWCAP / 64];
-#pragma unroll
-        for (int i = 0; i < (int)(TWCAP / 64); ++i) {
-          const uint32_t k = lane() + 64u * (uint32_t)i;
-          ev[i] = k < wn ? wc[k] : 0ull;
-          keep[i] = k < wn && (uint32_t)(ev[i] >> 32) >= lthr;
-        }
-        uint32_t mk = 0;
-#pragma unroll
-        for (int i = 0; i < (int)(TWCAP / 64); ++i) {
-          const uint64_t b = __builtin_amdgcn_ballot_w64(keep[i]);
-          if (keep[i]) wc[mk + lanes_below(b)] = ev[i];
-          mk += (uint32_t)__builtin_popcountll(b);
-        }
-        if (lane() == 0) S.wkept[wave()] = mk;
-      }
-      lds_barrier();
+      // ---- the candidates ranked by counting (keys are distinct)
       uint32_t kb[TNW + 1];
       kb[0] = 0;
 #pragma unroll
-      for (int w = 0; w < TNW; ++w) kb[w + 1] = kb[w] + S.wkept[w];
+      for (int w = 0; w < TNW; ++w) kb[w + 1] = kb[w] + S.wcnt[w];
       for (uint32_t j = tid; j < kb[TNW]; j += TNT) {
         uint32_t w = 0;
 #pragma unroll
@@ -410,9 +464,6 @@ __global__ __launch_bounds__(TNT, 6) void topn_kernel(TopnArgs A) {
       exact_list<In>(A.list + ((uint64_t)row * A.C + chunk) * n, S, src, c0, c1, take, sup);
       listed = take;
     }
-    lds_barrier();
-#pragma unroll
-    for (int w = 0; w < TNW; ++w) sum += S.red_d[w];
   }
   if (tid == 0) {
     TopnStat* st = &A.stat[(uint64_t)row * A.C + chunk];
@@ -445,11 +496,28 @@ struct alignas(16) MergeSmem {
 };
 
 // The `want` largest of S.dense[0, m) (distinct keys, want <= m, want <=
-// TOPN_MAX) into S.top[0, want), sorted descending: a radix select of the
-// want-th largest high word (the f32 key), the entries above it, and the
-// ties at it by counting on the full key.
+// TOPN_MAX) into S.top[0, want), sorted descending.  Up to one entry per
+// thread (ordinary rows: about n to 2n): each entry's rank by counting, one
+// broadcast LDS read per other entry and one barrier.  More (near-ties): a
+// radix select of the want-th largest high word (the f32 key), the entries
+// above it, and the ties at it by counting on the full key; its passes'
+// barriers cost an ordinary row more than the counting.
 __device__ __forceinline__ void top_of_dense(MergeSmem& S, uint32_t m, uint32_t want) {
   const uint32_t tid = threadIdx.x;
+  if (m <= (uint32_t)TNT) {   // m is uniform over the workgroup
+    const unsigned long long e = tid < m ? S.dense[tid] : 0ull;
+    uint32_t r = 0;
+    if (tid < m) {
+      uint32_t i = 0;
+      for (; i + 8u <= m; i += 8u)
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) r += S.dense[i + k] > e ? 1u : 0u;
+      for (; i < m; ++i) r += S.dense[i] > e ? 1u : 0u;
+      if (r < want) S.top[r] = e;
+    }
+    __syncthreads();
+    return;
+  }
   constexpr int RM = (int)(MDCAP / TNT);
   if (tid == 0) { S.s_sel = 0u; S.s_tie = 0u; }
   if (want < m) {
@@ -501,6 +569,23 @@ __global__ __launch_bounds__(TNT) void topn_merge_kernel(TopnArgs A) {
   const uint32_t C = A.C;
   const unsigned long long* lists = A.list + (uint64_t)row * C * n;
   auto cnt_of = [&](uint32_t q) { return min(n, min(TCH, V - q * TCH)); };
+  // The first round's lists, loaded into registers before anything waits on
+  // the statistics: the merge is a chain of memory latencies, and this takes
+  // one (or several, a load per round of the workgroup) out of it.
+  const uint32_t grp = n > 0 ? (MDCAP - TOPN_MAX) / n : 0u;   // lists per round
+  const uint32_t mg = n > 0 ? ((1u << 20) + n - 1u) / n : 0u; // j / n == (j * mg) >> 20 for j < 2^14
+  constexpr int RP = (int)(MDCAP / TNT);
+  unsigned long long pre[RP];
+  {
+    const uint32_t span = min(C, grp) * n;   // <= MDCAP
+#pragma unroll
+    for (int i = 0; i < RP; ++i) {
+      const uint32_t j = tid + (uint32_t)i * TNT;
+      const uint32_t l = (j * mg) >> 20;
+      const bool in = j < span && j - l * n < cnt_of(l);
+      pre[i] = in ? __builtin_bit_cast(unsigned long long, ld_dev(reinterpret_cast<const double*>(&lists[j]))) : 0ull;
+    }
+  }
   // chunk statistics and the last entry of each full list (chunks tid, tid + TNT)
   float cm[2];
   double cs[2];
@@ -560,8 +645,6 @@ __global__ __launch_bounds__(TNT) void topn_merge_kernel(TopnArgs A) {
   if (lane() == 0) S.red_d[wave()] = rpart;
   uint32_t nrun = 0;
   if (n > 0) {
-    const uint32_t grp = (MDCAP - TOPN_MAX) / n;          // lists per round
-    const uint32_t mg = ((1u << 20) + n - 1u) / n;        // j / n == (j * mg) >> 20 for j < 2^14
     for (uint32_t q0 = 0; q0 < C; q0 += grp) {
       const uint32_t q1 = min(C, q0 + grp);
       if (tid == 0) S.s_m = 0u;
@@ -572,7 +655,13 @@ __global__ __launch_bounds__(TNT) void topn_merge_kernel(TopnArgs A) {
         const unsigned long long e = S.top[j];
         if (e >= thr) S.dense[atomicAdd(&S.s_m, 1u)] = e;
       }
-      const uint32_t span = (q1 - q0) * n;
+      if (q0 == 0u) {
+        // (a missing entry is 0: an entry's low word is ~id, never 0)
+#pragma unroll
+        for (int i = 0; i < RP; ++i)
+          if (pre[i] != 0ull && pre[i] >= thr) S.dense[atomicAdd(&S.s_m, 1u)] = pre[i];
+      }
+      const uint32_t span = q0 == 0u ? 0u : (q1 - q0) * n;
       for (uint32_t j = tid; j < span; j += TNT) {
         const uint32_t l = (j * mg) >> 20;
         const uint32_t pos = j - l * n;

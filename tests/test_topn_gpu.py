@@ -124,3 +124,18 @@ def test_bf16_and_nonfinite(torch_mod, sampler, orc):
     bits[4, 5] = 0x7f80       # +inf
     x = synth.bf16_bits_to_f32(bits)
     check(torch_mod, sampler, orc, x, 28, bf16_bits=bits, name="bf16")
+
+
+# The unshifted weights' range (lane maxima up to 80; below 0 only with a lane
+# minimum above -86) and each way out of it, on both sides of every edge, in a
+# chunk's remainder and in a whole one; 9000 leaves a chunk of less than one
+# slice whose last wave holds fewer lanes than its share of n.  The
+# log-normalizer's derived bound is check()'s: 2^-22.
+@pytest.mark.parametrize("top", [-300.0, -86.5, -85.0, -1e-6, 0.0, 3e-7, 20.0, 79.9, 80.0, 80.1, 700.0])
+@pytest.mark.parametrize("V,n", [(8192, 20), (8197, 20), (9000, 64)])
+def test_weight_ranges(torch_mod, sampler, orc, top, V, n):
+    rng = np.random.default_rng(int(abs(top) * 10) + V)
+    x = (top - np.abs(rng.standard_normal((6, V)) * [[0.1], [3.0], [30.0], [3.0], [3.0], [0.0]])).astype(np.float32)
+    x[3, 5:] -= np.float32(95.0)        # all but five tokens near or below f32's normal range relative to the maximum
+    x[4, ::3] = -3e38                   # far below every weight's range
+    check(torch_mod, sampler, orc, x, n, name=f"top {top} V {V}")
