@@ -368,13 +368,15 @@ __global__ __launch_bounds__(TNT, 6) void topn_kernel(TopnArgs A) {
   // rounding of a value 2^-24 as large).  It may where no lane's maximum passes
   // 80 (e^80 in f32 range) and no weight falls below f32's normal range that
   // would not relative to the lane maximum too: a maximum >= 0, or a minimum
-  // above -86.  The weights are summed in f64, the corrections w r (2^-24 as
-  // large) in f32, which rounds 2^-48 of the lane's sum away; the maximum's
-  // own weight is then taken out of the sum again (the same instructions give
-  // the same bits) and enters as exactly 1.  A wave with a lane whose other
-  // tokens together weigh less than 2^-20 of its maximum, where 2^-48 of the
-  // maximum would show, takes the f64 differences.  Logits below -200
-  // (out-of-range and suppressed tokens too) weigh 0.
+  // above -86.  The residual r is below 2^-18 (half an ulp of yh < 128).  The
+  // weights are summed in f64, the corrections w r in f32; the maximum's own
+  // weight is then taken out of the sum again (the same instructions give the
+  // same bits) and enters as exactly 1.  The f32 sum holds the maximum's own
+  // correction too, so each of its 32 steps rounds by up to 2^-42 of the
+  // maximum: a wave with a lane whose other tokens together weigh less than
+  // 2^-13 of its maximum, where those 2^-37 would pass 2^-24 of their weight,
+  // takes the f64 differences (a lane maximum 9 nats above the rest: rare).
+  // Logits below -200 (out-of-range and suppressed tokens too) weigh 0.
   bool direct = __builtin_amdgcn_ballot_w64(t1 > -INFINITY && !(t1 >= 0.0f && t1 <= 80.0f)) == 0ull;
   if (!direct) {
     float tmin = INFINITY;
@@ -396,7 +398,7 @@ __global__ __launch_bounds__(TNT, 6) void topn_kernel(TopnArgs A) {
       }
     const float w1 = exp_f32r(t1, &r);
     part = (part - (double)w1) + ((double)corr - (double)w1 * (double)r);   // the lane's tokens but its maximum
-    direct = __builtin_amdgcn_ballot_w64(t1 > -INFINITY && !(part >= (double)w1 * 0x1p-20)) == 0ull;
+    direct = __builtin_amdgcn_ballot_w64(t1 > -INFINITY && !(part >= (double)w1 * 0x1p-13)) == 0ull;
     if (!direct) part = 0.0;
   }
   if (!direct && t1 > -INFINITY) {

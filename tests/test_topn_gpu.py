@@ -139,3 +139,36 @@ def test_weight_ranges(torch_mod, sampler, orc, top, V, n):
     x[3, 5:] -= np.float32(95.0)        # all but five tokens near or below f32's normal range relative to the maximum
     x[4, ::3] = -3e38                   # far below every weight's range
     check(torch_mod, sampler, orc, x, n, name=f"top {top} V {V}")
+
+
+# One lane of a chunk (tokens 1024 q + 0..3 of thread 0) holds its maximum and
+# `cnt` tokens that weigh 2^k of it together; everything else weighs nothing.
+# The top token's log probability is then -ln(1 + 2^k): its relative error is
+# that of the lane's other weights, 2^-22 at most, on both sides of the bar
+# (2^-13) below which the lane takes the f64 differences.  2^-30 covers the f64
+# sums and logs.
+@pytest.mark.parametrize("top", [5.0, 42.0, 60.0, 79.9])
+def test_lane_just_below_its_maximum(torch_mod, sampler, top):
+    rng = np.random.default_rng(int(top))
+    lane = np.array([1024 * q + e for q in range(8) for e in range(4)])
+    rows = []
+    for k in (-19.9, -18.0, -16.0, -14.0, -13.1, -12.9, -12.0, -10.0):
+        for cnt in (1, 4, 31):
+            for first in (True, False):
+                x = np.full(8192, top - 60.0, dtype=np.float32)
+                t = np.float32(top - rng.uniform(0.0, 3.0))
+                o = t - (np.log(cnt) - k * np.log(2.0)) + 1e-3 * rng.standard_normal(cnt)
+                vals = [t, *o] if first else [*o, t]
+                x[lane[:cnt + 1]] = np.array(vals, dtype=np.float32)
+                rows.append(x)
+    x = np.stack(rows)
+    say(f"case lane-below-maximum: rows {x.shape[0]} vocab 8192 top {top}")
+    ids, lps, mx, ln, st = (a.cpu().numpy() for a in sampler.logsoftmax_topn(upload(torch_mod, x), 8, vocab=8192))
+    assert (st == 0).all()
+    at = np.arange(len(x)), x.argmax(1)
+    d = x.astype(np.float64) - x[at].astype(np.float64)[:, None]
+    d[at] = -np.inf
+    want = -np.log1p(np.exp(d).sum(1))
+    assert (ids[:, 0] == at[1]).all()
+    err = np.abs(lps[:, 0] - want) / np.abs(want)
+    assert err.max() <= 2.0 ** -22 + 2.0 ** -30, (top, float(np.log2(err.max())), int(err.argmax()))
