@@ -255,16 +255,16 @@ struct RowCfg {
 // the compiler reads them with scalar loads (uniform per workgroup).  The
 // host substitutes default arrays for the ABI's NULLs, so none is null here.
 struct RowParams {
-  const double* __restrict__ temperature;
-  const uint32_t* __restrict__ top_k;
-  const double* __restrict__ top_p;
-  const double* __restrict__ min_p;
-  const float* __restrict__ repetition;
-  const float* __restrict__ presence;
-  const float* __restrict__ frequency;
-  const double* __restrict__ uniform;
-  const uint32_t* __restrict__ history_offsets;
-  const uint32_t* __restrict__ bias_offsets;
+  const double* temperature;
+  const uint32_t* top_k;
+  const double* top_p;
+  const double* min_p;
+  const float* repetition;
+  const float* presence;
+  const float* frequency;
+  const double* uniform;
+  const uint32_t* history_offsets;
+  const uint32_t* bias_offsets;
 };
 
 __device__ __forceinline__ RowCfg load_cfg(const double* __restrict__ temperature, const uint32_t* __restrict__ top_k,
@@ -3238,13 +3238,13 @@ __device__ __forceinline__ uint32_t reduce_head(const float* cand_l, const uint3
   return res;
 }
 
-// `nuc_row`: a top-p row (no top-k, no min-p) whose chunks listed their nucleus
+// NUC: a top-p row (no top-k, no min-p) whose chunks listed their nucleus
 // candidates and their whole mass; returns true when the row has to be
 // finished over every legal token instead (the nucleus may reach below what
 // every chunk lists, or the f32 part of the mass left a cut uncertified).
-template <typename In>
+template <typename In, bool NUC>
 __device__ __forceinline__ bool finish_row(const SampleArgs& A, FinSmem& F, const RowCfg& c, uint32_t row, uint32_t mode,
-                           uint64_t rbase, double invT, const FinLoads& P, const bool nuc_row) {
+                           uint64_t rbase, double invT, const FinLoads& P) {
   const mxs_batch& b = A.b;
   const uint32_t tid = threadIdx.x;
   const uint32_t V = b.vocab;
@@ -3279,7 +3279,7 @@ __device__ __forceinline__ bool finish_row(const SampleArgs& A, FinSmem& F, cons
     const uint32_t qmax = wave_max_u32(v.ncand);
     // the smallest candidate threshold (order keys; chunks without candidates do not count)
     const uint32_t lokey = ~wave_max_u32(v.ncand ? ~okey(v.thr) : 0u);
-    const uint32_t tlo = nuc_row ? wave_max_u32(v.nlegal ? okey(v.thr) : 0u) : 0u;
+    const uint32_t tlo = NUC ? wave_max_u32(v.nlegal ? okey(v.thr) : 0u) : 0u;
     // the greedy argmax: largest (value key, ~id); chunk values are +0.0-normalised
     const unsigned long long garg = wave_max_u64(
         v.gbest_id != NONE ? ((unsigned long long)okey(v.gbest_val) << 32) | (unsigned long long)(~v.gbest_id) : 0ull);
@@ -3333,7 +3333,7 @@ __device__ __forceinline__ bool finish_row(const SampleArgs& A, FinSmem& F, cons
   X.nodraw = A.nodraw != 0u;
   // (chunks that list every legal token: their sum is the row's, as for any
   // all-candidates row)
-  const bool nuc = nuc_row && okey_value(F.hdr.tlo) > -INFINITY;
+  const bool nuc = NUC && okey_value(F.hdr.tlo) > -INFINITY;
   X.nuc = nuc;
   X.stw = &F.hdr.st;
   if (err) {
@@ -3586,7 +3586,7 @@ __device__ __forceinline__ bool finish_row(const SampleArgs& A, FinSmem& F, cons
   // top_p of the row's.  f32 weights: relative error below 1e-5 (three
   // roundings of an exponent of at most 126 octaves and 2 ulp of exp2); a
   // mass within 4e-5 of the bar counts as below it.
-  if (nuc_row && !X.lds_c) return true;
+  if (NUC && !X.lds_c) return true;
   const bool short_row = ((mode == M_TOPK && c.k <= 64u) || mode == M_MINP) && ncand > 0u &&
                          ncand <= (uint32_t)(WR * 64) && X.lds_c;
   if (short_row || nuc) {
@@ -6001,12 +6001,9 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
   stamp(A, row, chunk, 5);
   if (emit || mass32 || mass64) lds_barrier();
   if (mass32 || mass64) {
-    // (thread 0 publishes the mass: wave 0 combines the waves' sums)
     double s0 = 0.0, s1 = 0.0;
-    if (wave() == 0) {
-      s0 = wave_sum_f64(lane() < (uint32_t)NW ? S.wq[lane()].m0 : 0.0);
-      s1 = mass32 ? wave_sum_f64(lane() < (uint32_t)NW ? S.wq[lane()].m1 : 0.0) : 0.0;
-    }
+#pragma unroll
+    for (int w = 0; w < NW; ++w) { s0 += S.wq[w].m0; s1 += S.wq[w].m1; }
     mass = s0;
     if (mass32) {
       // |mass - sum of exact weights| <= 1.01 (2^-22 S + 3 2^-24 S) for the
@@ -6032,9 +6029,11 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
     ncand = t0 + t1s + t2s;
     const uint32_t x0 = i0 - v0, x1 = i1 - v1 + t0, x2 = i2 - v2 + t0 + t1s;
     const uint64_t cbase = rbase + c0;
-    // as the lean body: staged in LDS (the count tables are dead by now),
-    // then copied out with coalesced stores
-    const bool staged = ncand <= (uint32_t)(CHUNK_MAX / 4);   // uniform
+    // nucleus rows, as the lean body: staged in LDS (the count tables are dead
+    // by now), then copied out with coalesced stores.  The other rows list few
+    // tokens per chunk, and the barrier costs them more than the stores (64
+    // rows with a bias list, top-k 20: 38.1 -> 41.3 us per call).
+    const bool staged = NUC && ncand <= (uint32_t)(CHUNK_MAX / 4);   // uniform
     float* stl = reinterpret_cast<float*>(S.t.ct);
     uint32_t* sti = S.t.ct + CHUNK_MAX / 4;
     double cpart = 0.0;   // nucleus rows: this thread's share of the candidates' mass
@@ -6157,6 +6156,80 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
 // row's parameters decide the body: rows the lean body covers issue the
 // history ids and the stream there and run it, the others run the general
 // body (which issues its own loads).
+// The nucleus rows' part of the kernel reads its arguments again, from the
+// kernel's argument segment, laid out as below: with the arguments the other
+// rows hold in registers, its chunk body and whole-row finish made those spill
+// (SGPR spills 209 -> 284; the other modes 1 to 3% slower).
+struct SampleKernArgs {
+  SampleArgs A;
+  RowParams P;
+};
+static_assert(sizeof(SampleArgs) % 8 == 0 && offsetof(SampleKernArgs, P) == sizeof(SampleArgs),
+              "the by-value arguments and the pointers behind them follow each other");
+typedef const SampleKernArgs __attribute__((address_space(4)))* KernArgs;
+
+// (a pointer read from memory is generic: the compiler would take flat
+// instructions for it, which wait on LDS and global loads alike)
+template <typename T>
+__device__ __forceinline__ void global_ptr(T*& p) {
+  p = (T*)(__attribute__((address_space(1))) T*)p;
+}
+// (read only while the kernel runs: scalar loads)
+template <typename T>
+__device__ __forceinline__ void const_ptr(const T*& p) {
+  p = (const T*)(const __attribute__((address_space(4))) T*)p;
+}
+// (opaque: a second read of an argument, not the kernel's own)
+__device__ __forceinline__ KernArgs kern_args() {
+  KernArgs k = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  __asm__ volatile("" : "+s"(k));
+  return k;
+}
+__device__ __forceinline__ SampleArgs load_args(KernArgs k) {
+  SampleArgs A = *(const SampleArgs*)&k->A;
+  global_ptr(A.b.logits); global_ptr(A.b.history_ids); global_ptr(A.b.bias_ids); global_ptr(A.b.bias_values);
+  global_ptr(A.b.mask_words);
+  global_ptr(A.o.token); global_ptr(A.o.sampling_logprob); global_ptr(A.o.status); global_ptr(A.o.kept_count);
+  global_ptr(A.o.adjusted); global_ptr(A.o.kept_bits);
+  global_ptr(A.w.ctr); global_ptr(A.w.rowx); global_ptr(A.w.stat); global_ptr(A.w.cand_l); global_ptr(A.w.cand_id);
+  global_ptr(A.w.adj); global_ptr(A.w.seg); global_ptr(A.w.cand_rows);
+  global_ptr(A.timing); global_ptr(A.paths); global_ptr(A.race_m);
+  return A;
+}
+__device__ __forceinline__ RowCfg load_cfg(KernArgs k, uint32_t row) {
+  RowParams p = *(const RowParams*)&k->P;
+  const_ptr(p.temperature); const_ptr(p.top_k); const_ptr(p.top_p); const_ptr(p.min_p); const_ptr(p.repetition);
+  const_ptr(p.presence); const_ptr(p.frequency); const_ptr(p.uniform); const_ptr(p.history_offsets);
+  const_ptr(p.bias_offsets);
+  return load_cfg(p.temperature, p.top_k, p.top_p, p.min_p, p.repetition, p.presence, p.frequency, p.uniform,
+                  p.history_offsets, p.bias_offsets, row);
+}
+
+// A nucleus row's chunk.
+template <typename In>
+__device__ __forceinline__ void nuc_chunk(FusedSmem& U, uint32_t row, uint32_t chunk) {
+  const KernArgs k = kern_args();
+  const SampleArgs A = load_args(k);
+  const RowCfg c = load_cfg(k, row);
+  chunk_general<In, true>(A, U, c, row, chunk, false);
+}
+
+// A nucleus row's finish: over its candidates, or over the whole row where they
+// do not decide it.
+template <typename In>
+__device__ __forceinline__ void nuc_finish(FinSmem& F, uint32_t row) {
+  const KernArgs k = kern_args();
+  const SampleArgs A = load_args(k);
+  const RowCfg c = load_cfg(k, row);
+  const double invT = 1.0 / c.T;
+  FinLoads P;
+  fin_issue(A, row, P);
+  if (finish_row<In, true>(A, F, c, row, M_ALL, (uint64_t)row * A.b.vocab, invT, P)) {
+    __syncthreads();   // the finisher's LDS is free
+    finish_nuc<In>(A, F, c, row, invT);
+  }
+}
+
 template <typename In, bool RX>
 __global__ __launch_bounds__(NT) void sample_kernel(
     SampleArgs A, const double* __restrict__ p_temperature, const uint32_t* __restrict__ p_top_k,
@@ -6178,6 +6251,7 @@ __global__ __launch_bounds__(NT) void sample_kernel(
   const uint32_t mode = chunk_mode(c, V);
   // a step receipt for this row (mxs_step)
   const bool rx = RX && A.rx_want[row] != MXS_RECEIPT_NONE;
+  const bool nuc = !c.err && nucleus_only(c, V);
   uint32_t rxw;   // the receipt work left after the body
   {
     const uint32_t hn = c.he > c.hb ? c.he - c.hb : 0u, bn = c.be > c.bb ? c.be - c.bb : 0u;
@@ -6204,8 +6278,12 @@ __global__ __launch_bounds__(NT) void sample_kernel(
         else rxw = chunk_fast<In, M_MINP, false, RX>(A, U, c, row, chunk, c0, c1, 0u, 0u, rx);
       }
     } else {
-      if (!c.err && nucleus_only(c, V)) rxw = chunk_general<In, true>(A, U, c, row, chunk, rx);
-      else rxw = chunk_general<In, false>(A, U, c, row, chunk, rx);
+      if (nuc) {
+        nuc_chunk<In>(U, row, chunk);
+        rxw = rx ? RX_FULL : 0u;
+      } else {
+        rxw = chunk_general<In, false>(A, U, c, row, chunk, rx);
+      }
     }
   }
   // The step receipt's reload paths run here, after the body, where its
@@ -6245,14 +6323,12 @@ __global__ __launch_bounds__(NT) void sample_kernel(
     return;
   }
   stamp(A, row, MAXC, 0);
-  FinLoads P;
-  fin_issue(A, row, P);
-  // (a nucleus row its candidates could not decide is finished over the
-  // whole row)
-  if (finish_row<In>(A, U.f, c, row, mode, (uint64_t)row * V, c.greedy ? 0.0 : 1.0 / c.T, P,
-                     !c.err && nucleus_only(c, V))) {
-    __syncthreads();   // the finisher's LDS is free
-    finish_nuc<In>(A, U.f, c, row, 1.0 / c.T);
+  if (nuc) {
+    nuc_finish<In>(U.f, row);
+  } else {
+    FinLoads P;
+    fin_issue(A, row, P);
+    finish_row<In, false>(A, U.f, c, row, mode, (uint64_t)row * V, c.greedy ? 0.0 : 1.0 / c.T, P);
   }
   stamp(A, row, MAXC, 7);
   if (RX && rx) {
@@ -6746,7 +6822,7 @@ __global__ __launch_bounds__(NT) void tile_finish_kernel(SampleArgs A, const Epi
   __syncthreads();
   FinLoads P;
   fin_issue(A, row, P);
-  finish_row<float>(A, U.f, c, row, mode, rbase, c.greedy ? 0.0 : 1.0 / c.T, P, false);
+  finish_row<float, false>(A, U.f, c, row, mode, rbase, c.greedy ? 0.0 : 1.0 / c.T, P);
 }
 
 }  // namespace mxs
