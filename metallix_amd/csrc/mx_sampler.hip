@@ -220,6 +220,7 @@ struct alignas(16) FinSmem {
     double L;                          // ln(min_p) (-inf for min_p = 0)
     uint32_t flags, nlegal, Mkey, bi, ncand;
     uint32_t qmax;                     // the largest candidate count of a chunk
+    uint32_t unsummed;                 // a nuc row's chunk lists all its tokens without their mass (mass_err = inf)
     float lo;                          // no candidate is below it (the chunks' smallest threshold)
     uint32_t tlo;                      // order key of the chunks' largest threshold (every legal token from it up is listed)
     uint32_t st;                       // a nuc row's status
@@ -326,11 +327,13 @@ __device__ __forceinline__ uint32_t chunk_mode(const RowCfg& c, uint32_t V) {
   return M_KEEPALL;
 }
 
-// Top-p alone (no active top-k, no min-p): the rows whose chunks list
-// nucleus candidates.  The other all-candidates rows (a top-k beyond
-// KCAND_MAX) list every legal token.
+// Top-p alone (no active top-k, no min-p) over a vocabulary the finisher's
+// cache does not hold: the rows whose chunks list nucleus candidates.  The
+// other all-candidates rows (a top-k beyond KCAND_MAX, a small vocabulary)
+// list every legal token; thinned lists cost a small vocabulary up to a tenth
+// more (32 x 2000 f32 26.9 -> 29.0 us per call, 32 x 5001 34.2 -> 35.6).
 __device__ __forceinline__ bool nucleus_only(const RowCfg& c, uint32_t V) {
-  return chunk_mode(c, V) == M_ALL && !(c.k > 0 && c.k < V);
+  return V > (uint32_t)CCAP && chunk_mode(c, V) == M_ALL && !(c.k > 0 && c.k < V);
 }
 
 // Logit-bias and penalty stage for one token (BUILD-DEFINED semantics, f32,
@@ -3306,7 +3309,13 @@ __device__ __forceinline__ bool finish_row(const SampleArgs& A, FinSmem& F, cons
     const uint32_t q = lane();
     const bool qa = q < C;
     const uint32_t nlg = P.v.nlegal, mxk = P.v.maxkey;
-    const double ms = P.v.mass, me = P.v.mass_err;
+    double ms = P.v.mass, me = P.v.mass_err;
+    if constexpr (NUC) {
+      const bool un = qa && me == INFINITY;
+      if (un) me = 0.0;   // (its mass is 0)
+      const uint64_t ub = __builtin_amdgcn_ballot_w64(un);
+      if (q == 0) F.hdr.unsummed = ub ? 1u : 0u;
+    }
     const uint32_t mkey = wave_max_u32(nlg ? mxk : 0u);
     const double Mw = (double)okey_value(mkey);
     const double cs = nlg ? exp_neg_p(((double)okey_value(mxk) - Mw) * invT) : 0.0;
@@ -3331,9 +3340,9 @@ __device__ __forceinline__ bool finish_row(const SampleArgs& A, FinSmem& F, cons
   X.cand_l = A.w.cand_l; X.cand_id = A.w.cand_id; X.CH = A.CH; X.o = A.o; X.c = c; X.row = row; X.mode = mode; X.C = C; X.V = V; X.nlegal = nlegal; X.rbase = rbase;
   X.kbits = kbits; X.nwords = nwords; X.M = M; X.timing = A.timing; X.paths = A.paths; X.etab = F.etab;
   X.nodraw = A.nodraw != 0u;
-  // (chunks that list every legal token: their sum is the row's, as for any
-  // all-candidates row)
-  const bool nuc = NUC && okey_value(F.hdr.tlo) > -INFINITY;
+  // (up to CCAP legal tokens: every chunk lists its own, and their sum is the
+  // row's, as for any all-candidates row)
+  const bool nuc = NUC && nlegal > (uint32_t)CCAP;
   X.nuc = nuc;
   X.stw = &F.hdr.st;
   if (err) {
@@ -3586,12 +3595,28 @@ __device__ __forceinline__ bool finish_row(const SampleArgs& A, FinSmem& F, cons
   // top_p of the row's.  f32 weights: relative error below 1e-5 (three
   // roundings of an exponent of at most 126 octaves and 2 ulp of exp2); a
   // mass within 4e-5 of the bar counts as below it.
-  if (NUC && !X.lds_c) return true;
+  if (nuc && !X.lds_c) return true;
   const bool short_row = ((mode == M_TOPK && c.k <= 64u) || mode == M_MINP) && ncand > 0u &&
                          ncand <= (uint32_t)(WR * 64) && X.lds_c;
   if (short_row || nuc) {
     if (!loaded) bulk_load();
     loaded = true;
+  }
+  if (nuc && F.hdr.unsummed) {
+    // the mass of the chunks that list all their tokens without it
+    double un = 0.0;
+    uint32_t qj = 0, nxt = C > 1 ? F.coff[1] : NONE;
+#pragma unroll
+    for (int u = 0; u < FR; ++u) {
+      const uint32_t j = (uint32_t)u * FT + tid;
+      if (j < ncand) {
+        while (j >= nxt) { ++qj; nxt = qj + 1 < C ? F.coff[qj + 1] : NONE; }
+        if (F.st[qj].mass_err == INFINITY) un += exp_neg_t(((double)F.cl[j] - M) / c.T, F.etab, F.etab + 64);
+      }
+    }
+    un = block_sum<double>(un, F.red_d);
+    X.total += un;
+    X.total_err += sum_bound(un, ncand + (uint32_t)FT, 8.0) + sum_bound(X.total, C, 8.0);
   }
   if (nuc) {
     const float Mf = (float)M, c2 = (float)(invT * 1.4426950408889634), tl = okey_value(F.hdr.tlo);
@@ -5757,21 +5782,50 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
   // finished over the whole row).  A token too far below the largest chunk
   // maximum published so far is no candidate either (nuc_reach).
   // A chunk of few legal tokens (grammar masks) packs them first, as a
-  // candidate list; beyond nuc_list of them it counts and thins that list,
-  // one to four entries per thread where the registers hold a few legal
-  // lanes per element.
-  // (A row of up to CCAP legal tokens has them spread over its chunks to
-  // within a half, and is decided best with all of them listed: thinning
-  // 6,000 to 7,400 legal tokens of flat bf16 rows left 90% and cost 4 us.
-  // Such chunks sum no mass; beside chunks that thin their lists it counts
-  // as unknown, which sends the row to finish_nuc.)
-  const uint32_t nuc_list = (uint32_t)CCAP / A.C * 3u / 2u;
-  const bool nuc_pack = NUC && emit && nleg <= 4u * (uint32_t)NT;
+  // candidate list.  Up to nuc_list of them stay listed without a mass (the
+  // finisher sums it where the others' masses count); beyond that the row's
+  // mask words are counted: a row of at most CCAP legal tokens lists them all
+  // (its finisher decides it from the LDS cache; thinned lists can miss the
+  // nucleus: with half of 3000 legal tokens of 151936 in one run, 32 rows took
+  // 128 instead of 37 us), the others' chunks count and thin the list, one to
+  // four entries per thread where the registers hold a few legal lanes per
+  // element.
+  const uint32_t nuc_list = min((uint32_t)CCAP / A.C * 3u / 2u, 4u * (uint32_t)NT);
+  bool nuc_all = false;
+  if (NUC && emit && masked_row) {
+    nuc_all = nleg <= nuc_list;
+    if (!nuc_all) {   // uniform
+      typedef uint32_t Words __attribute__((ext_vector_type(4), aligned(4)));
+      const uint32_t rlim = min(V, b.tokenizer_vocab), rfull = rlim >> 7;   // whole groups of 4 words
+      const uint32_t* rmp = b.mask_words + (uint64_t)row * b.mask_stride;
+      uint32_t rn = 0u;
+#pragma unroll 1
+      for (uint32_t g = tid; g < rfull; g += 2u * (uint32_t)NT) {
+        const Words a = *reinterpret_cast<const Words*>(rmp + 4u * g);
+        const uint32_t g2 = min(g + (uint32_t)NT, rfull - 1u);
+        const Words d = *reinterpret_cast<const Words*>(rmp + 4u * g2);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          rn += (uint32_t)__builtin_popcount(a[e]);
+          rn += g + (uint32_t)NT < rfull ? (uint32_t)__builtin_popcount(d[e]) : 0u;
+        }
+      }
+      // the last, partial group's bits, one per thread
+      const uint32_t rt = (rfull << 7) + tid;
+      if (tid < 128u && rt < rlim) rn += (rmp[rt >> 5] >> (rt & 31u)) & 1u;
+      rn = wave_sum_u32(rn);
+      if (lane() == 0) S.wq[wave()].nleg = rn;
+      lds_barrier();
+      rn = wave_sum_u32(lane() < (uint32_t)NW ? S.wq[lane()].nleg : 0u);
+      nuc_all = rn <= (uint32_t)CCAP;
+    }
+  }
+  const bool nuc_pack = NUC && emit && (nuc_all || nleg <= 4u * (uint32_t)NT);
   const bool nuc_x = NUC && emit && !nuc_pack;
   // The row maximum so far (every chunk publishes its own), waited for where
   // the threshold needs it.
   unsigned long long xold = 0ull;
-  if (NUC && emit && nleg > nuc_list && tid == 0)
+  if (NUC && emit && !nuc_all && tid == 0)
     xold = __hip_atomic_fetch_max(A.w.rowx + (uint64_t)row * ROWX_STRIDE, ((unsigned long long)A.epoch << 32) | maxkey,
                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   auto nuc_row_max = [&]() {
@@ -6073,7 +6127,7 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
         }
       }
     }
-    if (nuc_pack && nleg > nuc_list) {
+    if (nuc_pack && !nuc_all) {
       lds_barrier();
       const float hs = (float)(invT * 1.4426950408889634) * 32.0f;
       const uint32_t R = (ncand + (uint32_t)NT - 1u) / (uint32_t)NT, j0 = tid * R;
@@ -6107,8 +6161,8 @@ __device__ __forceinline__ uint32_t chunk_general(const SampleArgs& A, FusedSmem
         if (nuc_x) cpart += exp_neg_t(((double)l - md) * invT, S.etab, S.etab + 64);
       }
     }
-    if (nuc_pack && nleg <= nuc_list) mass_err = INFINITY;   // all listed, not summed
-    if (nuc_x || (nuc_pack && nleg > nuc_list)) {
+    if (NUC && nuc_all) mass_err = INFINITY;   // all listed, not summed
+    if (NUC && !nuc_all) {
       const double w0s = wave_sum_f64(m0), w1s = wave_sum_f64(m1), w2s = wave_sum_f64(cpart);
       if (lane() == 0) { S.wq[wave()].m0 = w0s; S.wq[wave()].m1 = w1s; S.wp[wave()].m0 = w2s; }
       lds_barrier();

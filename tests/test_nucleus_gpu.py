@@ -150,3 +150,42 @@ def test_paths(torch_mod, orc):
         assert ((got == LARGE) == large).all(), (kind, got)
     s.lib.mxs_debug_set_paths(s.ctx, None)
     s.close()
+
+
+def clustered(rng, R, V, total, share):
+    """Mask words with `total` legal tokens per row, `share` of them in one run."""
+    legal = np.zeros((R, (V + 31) // 32 * 32), dtype=bool)
+    run = int(total * share)
+    for r in range(R):
+        legal[r, rng.choice(V, total - run, replace=False)] = True
+        s = int(rng.integers(0, V - run + 1))
+        legal[r, s:s + run] = True
+    return np.packbits(legal.reshape(R, -1, 32), axis=-1, bitorder="little").view(np.uint32).reshape(R, -1)
+
+
+# Legal tokens that lie in few of a row's chunks: up to 8192 of them (the
+# finisher's cache) every chunk lists its own whatever its share, beyond that
+# every chunk thins its list and sums its mass.
+@pytest.mark.parametrize("kind", ["text", "flat"])
+@pytest.mark.parametrize("V,total,share", [(151936, 1000, 1.0), (151936, 3000, 0.55), (151936, 4000, 1.0), (151936, 8192, 0.9),
+                                           (151936, 9000, 0.5), (40000, 12000, 1.0), (262144, 3000, 0.55), (20011, 3500, 0.7), (20011, 10000, 0.5)])
+def test_clustered_masks(torch_mod, orc, kind, V, total, share):
+    from helpers import to_device
+    from metallix_amd import Sampler
+
+    R = 8
+    b = batch(kind, R, V, bf16=kind == "flat", seed=7)
+    b.top_p = np.array([0.05, 0.5, 0.8, 0.9, 0.95, 0.95, 0.99, 0.999])
+    b.mask_words, b.tokenizer_vocab = clustered(np.random.default_rng(total), R, V, total, share), V - 3
+    print(f"case nucleus clustered {kind} vocab {V} legal {total} share {share}", flush=True)
+    s = Sampler(max_rows=R, max_vocab=V)
+    compare(b, run_gpu(torch_mod, s, b), orc.sample_batch(b, debug=True))
+    if total <= 4000:   # ... and such rows stay within the finisher's LDS working set
+        buf = torch_mod.zeros(R, dtype=torch_mod.int32, device="cuda")
+        s.lib.mxs_debug_set_paths(s.ctx, buf.data_ptr())
+        logits, kw = to_device(torch_mod, b)
+        s.sample(logits, **kw)
+        torch_mod.cuda.synchronize()
+        assert (buf.cpu().numpy() != LARGE).all(), buf.cpu().numpy()
+        s.lib.mxs_debug_set_paths(s.ctx, None)
+    s.close()
