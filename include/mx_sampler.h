@@ -240,12 +240,12 @@ int mxs_step(mxs_ctx* ctx, const mxs_batch* batch, const mxs_race* race, const m
  * its first `rows` rows, queued on the context's stream behind that call:
  * the list the row's finisher chose from (every candidate at or above its
  * chunk's threshold; it holds the row's top-k head for a top-k row, its
- * min-p set for a min-p row and, for a top-p row decided from its list, its
- * nucleus), as adjusted logits (penalties, bias, mask
- * applied) with their token IDs, in token-ID order.  count[r] = the list's
+ * min-p set for a min-p row and its nucleus for a top-p row; every legal
+ * token of a top-p row with status 1), as adjusted logits (penalties, bias,
+ * mask applied) with their token IDs, in token-ID order.  count[r] = the list's
  * length when at most `width`; else its top `width` by (logit desc, ID asc)
  * and count[r] = width; -1 for a row with no list (greedy, keep-all, error
- * rows).  ids and logits are rows x width.  The settle of an uncertified
+ * rows, and certified top-p rows whose nucleus no list holds).  ids and logits are rows x width.  The settle of an uncertified
  * (status 1) top-k row with k <= width: sort by (logit desc, ID asc), keep
  * the first k, and apply the row's rule to them, as pick_from_candidates'
  * sample_top_k_candidates does; the row need not be read back.  A later

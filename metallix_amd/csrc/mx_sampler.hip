@@ -3881,6 +3881,7 @@ __device__ __forceinline__ void finish_nuc(const SampleArgs& A, FinSmem& F, cons
   // |a computed sum of n weights - the reference's|
   auto bound = [&](double v, uint32_t n) { return sum_bound(v, n + 64u, 8.0); };
   bool uncert = false;
+  if (tid == 0) A.w.cand_rows[row] = -1;   // not chosen from the chunks' lists
   if (A.paths && tid == 0) A.paths[row] = MXS_PATH_LARGE;
 
   // ---- 1: the mass bins ----------------------------------------------------
@@ -4164,10 +4165,23 @@ __device__ __forceinline__ void finish_nuc(const SampleArgs& A, FinSmem& F, cons
     }
   }
   __syncthreads();
+  if (F.s_u[4] && !A.nodraw) uncert = true;
+  // An uncertified row's candidates (mxs_export_candidates) are every legal
+  // token: its adjusted logits, NaN where not legal.  (Writing them for every
+  // row that comes here cost 3 to 15%.)
+  if (uncert) {
+    unsigned long long* ex = reinterpret_cast<unsigned long long*>(A.w.adj + (uint64_t)row * ((V + 3u) & ~3u));
+    if (tid == 0) A.w.cand_rows[row] = -2 - (int32_t)nlegal;
+    each([&](uint32_t j, uint32_t id0, const float* x, uint32_t lb) {
+      if (j >= nj || id0 >= V) return;
+      auto bits = [&](int e) { return (unsigned long long)((lb >> e) & 1u ? __float_as_uint(x[e]) : 0x7fc00000u); };
+      st_dev(ex + id0 / 2u, bits(0) | (bits(1) << 32));
+      st_dev(ex + id0 / 2u + 1u, bits(2) | (bits(3) << 32));
+    });
+  }
   if (tid == 0) {
     const uint32_t tok = F.s_u[3];
     const bool none = tok == NONE;
-    if (F.s_u[4] && !A.nodraw) uncert = true;
     A.o.token[row] = none ? -1 : (int32_t)tok;
     A.o.status[row] = none ? MXS_ROW_EMPTY_SUPPORT : (uncert ? MXS_ROW_UNCERTIFIED : 0);
     if (A.o.sampling_logprob) A.o.sampling_logprob[row] = none ? 0.0 : F.s_d[1] - log(S);
@@ -6517,7 +6531,9 @@ int sample_launch(mxs_ctx* ctx, const mxs_batch* b, const mxs_out* o, bool nodra
 }
 
 // ---------------------------------------------------------------------------
-// Candidate export (mxs_export_candidates): row r's candidate list from the
+// Candidate export (mxs_export_candidates): every legal token of an uncertified
+// top-p row finished over its whole row (cand_rows = -2 - their number: its
+// adjusted logits, NaN where not legal), else row r's candidate list from the
 // last mxs_sample / mxs_step call, chunk q's candidates at r V + q CH
 // (ncand of them, token-ID order), copied out whole when at most `width`,
 // else its top `width` by (logit desc, ID asc): a radix select of the
@@ -6532,10 +6548,11 @@ __global__ __launch_bounds__(NT) void cand_export_kernel(Work w, uint32_t C, uin
   __shared__ uint32_t s_u[2];
   const uint32_t row = blockIdx.x, tid = threadIdx.x;
   const int32_t n0 = w.cand_rows[row];
-  if (n0 < 0) {
+  if (n0 == -1) {
     if (tid == 0) count[row] = -1;
     return;
   }
+  const bool whole = n0 < -1;
   if (tid < 64u) {   // chunk offsets (C <= MAXC = 64)
     const uint32_t nq = tid < C ? w.stat[(uint64_t)row * MAXC + tid].ncand : 0u;
     const uint32_t inc = wave_scan_u32(nq);
@@ -6544,7 +6561,8 @@ __global__ __launch_bounds__(NT) void cand_export_kernel(Work w, uint32_t C, uin
     if (tid == 0) coff[C] = tot;
   }
   __syncthreads();
-  const uint32_t n = min((uint32_t)n0, coff[C]);
+  const uint32_t n = whole ? (uint32_t)(-2 - n0) : min((uint32_t)n0, coff[C]);
+  const uint32_t items = whole ? V : n;   // list positions to look at
   const uint64_t rbase = (uint64_t)row * V;
   // candidate j's position: the last chunk q < C with coff[q] <= j
   auto pos_of = [&](uint32_t j) -> uint64_t {
@@ -6555,9 +6573,21 @@ __global__ __launch_bounds__(NT) void cand_export_kernel(Work w, uint32_t C, uin
     }
     return rbase + (uint64_t)lo * CH + (j - coff[lo]);
   };
+  const float* adj = w.adj + (uint64_t)row * ((V + 3u) & ~3u);
+  auto item = [&](uint32_t j, float* l, uint32_t* id) -> bool {
+    if (whole) {
+      *l = ld_dev(&adj[j]);
+      *id = j;
+      return *l == *l;
+    }
+    const uint64_t p = pos_of(j);
+    *l = ld_dev(&w.cand_l[p]);
+    *id = ld_dev(&w.cand_id[p]);
+    return true;
+  };
   int32_t* oi = ids + (uint64_t)row * width;
   float* ol = logits + (uint64_t)row * width;
-  if (n <= width) {
+  if (n <= width && !whole) {
     for (uint32_t j = tid; j < n; j += NT) {
       const uint64_t p = pos_of(j);
       oi[j] = (int32_t)ld_dev(&w.cand_id[p]);
@@ -6566,13 +6596,18 @@ __global__ __launch_bounds__(NT) void cand_export_kernel(Work w, uint32_t C, uin
     if (tid == 0) count[row] = (int32_t)n;
     return;
   }
-  uint32_t prefix = 0u, need = width;   // the key's fixed high digits; members still to take at or below them
-  for (int d = 3; d >= 0; --d) {
+  // the key's fixed high digits, and members still to take at or below them
+  // (no key is 0: with no selection everything is above the prefix)
+  uint32_t prefix = 0u, need = width;
+  for (int d = n > width ? 3 : -1; d >= 0; --d) {
     if (tid < 256u) hist[tid] = 0u;
     __syncthreads();
     const uint32_t pm = d == 3 ? 0u : (0xffffffffu << (8 * (d + 1)));
-    for (uint32_t j = tid; j < n; j += NT) {
-      const uint32_t key = okey(ld_dev(&w.cand_l[pos_of(j)]));
+    for (uint32_t j = tid; j < items; j += NT) {
+      float l;
+      uint32_t id;
+      if (!item(j, &l, &id)) continue;
+      const uint32_t key = okey(l);
       if ((key & pm) == prefix) atomicAdd(&hist[(key >> (8 * d)) & 255u], 1u);
     }
     __syncthreads();
@@ -6593,20 +6628,16 @@ __global__ __launch_bounds__(NT) void cand_export_kernel(Work w, uint32_t C, uin
   }
   // keys above `prefix` (width - need of them), then the first `need` ties in ID order
   uint32_t base = 0u, tbase = 0u;
-  for (uint32_t j0 = 0; j0 < n; j0 += NT) {
+  for (uint32_t j0 = 0; j0 < items; j0 += NT) {
     const uint32_t j = j0 + tid;
     uint32_t key = 0u, id = 0u;
     float l = 0.0f;
-    if (j < n) {
-      const uint64_t p = pos_of(j);
-      l = ld_dev(&w.cand_l[p]);
-      id = ld_dev(&w.cand_id[p]);
-      key = okey(l);
-    }
-    const bool tie = j < n && key == prefix;
+    const bool in = j < items && item(j, &l, &id);
+    if (in) key = okey(l);
+    const bool tie = in && key == prefix;
     uint32_t ttot;
     const uint32_t trank = tbase + block_scan_incl<uint32_t>(tie ? 1u : 0u, red, &ttot) - (tie ? 1u : 0u);
-    const bool take = (j < n && key > prefix) || (tie && trank < need);
+    const bool take = (in && key > prefix) || (tie && trank < need);
     uint32_t tot;
     const uint32_t at = base + block_scan_incl<uint32_t>(take ? 1u : 0u, red, &tot) - (take ? 1u : 0u);
     if (take && at < width) {

@@ -60,9 +60,11 @@ struct Work {
   ChunkStat* stat;            // [max_rows * MAXC]
   float* cand_l;              // [max_rows * max_vocab]
   uint32_t* cand_id;          // [max_rows * max_vocab]
-  float* adj;                 // [max_rows * roundup4(max_vocab)] adjusted logits of top-p rows with penalties or biases
+  float* adj;                 // [max_rows * roundup4(max_vocab)] adjusted logits: of top-p rows with penalties or
+                              // biases, and of uncertified ones finished over the whole row (NaN where not legal)
   double* seg;                // [max_rows * MAXC * PER_MAX * NW]
-  int32_t* cand_rows;         // [max_rows] candidates the row's finisher chose from (-1: no list)
+  int32_t* cand_rows;         // [max_rows] candidates the row's finisher chose from (-1: no list; -2 - n: the
+                              // row's n legal tokens, in adj)
 };
 
 }  // namespace mxs

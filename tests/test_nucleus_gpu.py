@@ -189,3 +189,46 @@ def test_clustered_masks(torch_mod, orc, kind, V, total, share):
         assert (buf.cpu().numpy() != LARGE).all(), buf.cpu().numpy()
         s.lib.mxs_debug_set_paths(s.ctx, None)
     s.close()
+
+
+@pytest.mark.parametrize("opt", [{}, dict(bf16=True, mask=True), dict(history=300, bias=5), dict(history=40, mask=True)],
+                         ids=lambda v: "-".join(v) or "plain")
+def test_export_of_top_p_rows(torch_mod, orc, opt):
+    """What a top-p row exports: a list that holds its nucleus where the chunks'
+    candidates decided it, none where the whole row did, and every legal token
+    (or the top `width` of them, ties by ID) of an uncertified row.  Rows 2 and 3
+    are flat; row 3's top_p puts the cut among weights below the f64 sums'
+    error bound, so it is uncertified."""
+    from metallix_amd import Sampler
+
+    R, V = 4, 40003
+    b = batch("text", R, V, seed=11, **opt)
+    flat = batch("flat", R, V, seed=11, **opt)
+    b.logits[2:] = flat.logits[2:]
+    if b.bf16_bits is not None:
+        b.bf16_bits[2:] = flat.bf16_bits[2:]
+    b.temperature, b.top_p = np.full(R, 0.8), np.array([0.5, 0.6, 0.999, 1.0 - 1e-15])
+    ref = orc.sample_batch(b, debug=True)
+    legal = np.ones((R, V), dtype=bool)
+    if b.mask_words is not None:
+        legal = np.unpackbits(b.mask_words.view(np.uint8), axis=1, bitorder="little")[:, :V].astype(bool)
+        legal[:, b.tokenizer_vocab:] = False
+    print(f"case export vocab {V} {opt}", flush=True)
+    s = Sampler(max_rows=R, max_vocab=V)
+    gpu = run_gpu(torch_mod, s, b)
+    assert list(gpu["status"]) == [0, 0, 0, 1], gpu["status"]
+    compare(b, gpu, ref, allow_uncertified=1)
+    for width in (V, 3000):
+        cnt, ids, lg = (t.cpu().numpy() for t in s.export_candidates(R, width))
+        assert cnt[2] == -1
+        for r in (0, 1, 3):
+            i, l = ids[r, :cnt[r]], lg[r, :cnt[r]]
+            assert np.array_equal(l.view(np.uint32), ref["adjusted"][r][i].view(np.uint32)) and legal[r, i].all()
+            assert (np.diff(i) > 0).all()
+            if r == 3:
+                all_ids = np.nonzero(legal[r])[0]
+                order = np.lexsort((all_ids, -ref["adjusted"][r][all_ids].astype(np.float64)))[:width]
+                assert np.array_equal(i, np.sort(all_ids[order])), (width, len(i))
+            elif width == V:
+                assert np.isin(np.nonzero(ref["kept"][r])[0], i).all()
+    s.close()
