@@ -23,8 +23,8 @@
 // (about 2^-50 (1 + |g| + |score|) each); otherwise the row's status is 1
 // (uncertified) and it carries the device's winner.
 //
-// Launch: rows * C workgroups of RNT threads; chunk c of a row covers tokens
-// [c RT, (c + 1) RT), RPT / 2 token pairs 2 RNT tokens apart per thread.
+// Launch: rows * C workgroups of RNT threads; chunk c of a row covers RT = RNT
+// RPT tokens from c RT on, RPT / 2 token pairs 2 RNT tokens apart per thread.
 // Each chunk reduces its kept tokens to a RaceStat; the row's last chunk to
 // arrive (device-scope counter) merges them and writes the row's result.
 #include <hip/hip_runtime.h>
@@ -38,9 +38,15 @@ namespace mxs {
 
 constexpr int RNT = 256;                       // threads per race workgroup
 constexpr int RNW = RNT / 64;
-constexpr uint32_t RPT = 16;                    // tokens per thread
-constexpr uint32_t RT = (uint32_t)RNT * RPT;    // tokens per race chunk
-constexpr uint32_t RKW = RT / 32u;              // kept-set words per chunk
+// Tokens per thread: 16, or 32 where the short chunks' workgroups would pass
+// RWIDE.  Most workgroups of rows under ordinary rules find no kept token and
+// cost their parameter loads and their arrival; the short chunks balance few
+// whole-row races better.  f32, V 151936, 16 / 32 tokens, us per call: 256 rows
+// under the serving rules with 2048 history IDs 143.9 / 133.2, all whole-row
+// races 236.7 / 223.0; 64 rows 48.4 / 45.9, half of them whole-row races 70.6 /
+// 72.5; one whole-row race 35.6 / 42.8.
+constexpr uint32_t RPT_SHORT = 16, RPT_WIDE = 32;
+constexpr uint32_t RWIDE = 4096;
 
 // One chunk's kept tokens, reduced.
 struct alignas(16) RaceStat {
@@ -57,6 +63,7 @@ constexpr uint32_t RF_ANY = 1u;        // the chunk keeps a token
 constexpr uint32_t RF_NONFINITE = 2u;  // a kept token's score is not finite
 
 size_t race_scratch_bytes(uint32_t max_rows, uint32_t max_vocab) {
+  constexpr uint32_t RT = (uint32_t)RNT * RPT_SHORT;
   return (size_t)max_rows * ((max_vocab + RT - 1u) / RT) * sizeof(RaceStat);
 }
 
@@ -176,7 +183,7 @@ __device__ __forceinline__ void best_merge(Best& a, double s1, double s2, uint32
 }
 
 // History counts of a chunk's tokens, two 16-bit counts per LDS word (token
-// d of the chunk in half d & 1), so that the table takes 16 KB and eight
+// d of the chunk in half d & 1), so that the table takes 8 or 16 KB and eight
 // workgroups share a CU.  A row with at most 65535 history entries cannot
 // carry a count into its neighbour, and plain adds are exact.  A longer
 // history adds with compare-and-swap, saturating at 0xFFFF, and a saturated
@@ -236,7 +243,10 @@ struct Pair<uint16_t> {
   }
 };
 
+template <uint32_t RPT>
 struct RaceSmem {
+  static constexpr uint32_t RT = (uint32_t)RNT * RPT;   // tokens per chunk
+  static constexpr uint32_t RKW = RT / 32u;             // its kept-set words
   uint32_t cnt[RT / 2];      // history counts of the chunk's tokens (16-bit pairs)
   float redf2[RNW];
   double redd[RNW];
@@ -247,9 +257,10 @@ struct RaceSmem {
   uint32_t any, last;
 };
 
-template <typename In>
+template <typename In, uint32_t RPT>
 __global__ __launch_bounds__(RNT) void race_kernel(RaceArgs A) {
-  __shared__ RaceSmem S;
+  __shared__ RaceSmem<RPT> S;
+  constexpr uint32_t RT = RaceSmem<RPT>::RT, RKW = RaceSmem<RPT>::RKW;
   // Workgroups in (row, chunk) order: workgroup i runs on XCD i mod 8, so a
   // row's chunks spread over the XCDs.  A whole-row race is compute (about
   // 450 cycles per 64 tokens), its chunks share only the kept words and the
@@ -320,7 +331,7 @@ __global__ __launch_bounds__(RNT) void race_kernel(RaceArgs A) {
       const bool hasb = lo < be && A.bids[lo] == id;
       return penalize_logit(l, cnt, hasb, hasb ? A.bvals[lo] : 0.0f, rep, pres, freq);
     };
-    // Thread tid takes the chunk's token pairs tid + RNT j (j < 8): the two
+    // Thread tid takes the chunk's token pairs tid + RNT j (j < RPT / 2): the two
     // tokens of a pair share one Philox block (race.rs:66-80), and a wave's
     // loads are 128 consecutive tokens.  Bits 2 j and 2 j + 1 of `mine` are
     // pair tid + RNT j's kept bits.
@@ -346,6 +357,29 @@ __global__ __launch_bounds__(RNT) void race_kernel(RaceArgs A) {
     uint64_t bits1 = 0ull;
     ExpCoef expo;
     expo.load();
+    auto score = [&](uint32_t id, float l, uint32_t hi, uint32_t lo) {
+      mass += expo(((double)l - (double)m) * invT);   // (within ulps of the quotient: the mass feeds only the logprob)
+      const float s32 = (l - m) * invT32 + gumbel32(hi, lo);
+      if (s32 > t1) {
+        t2 = t1; t1 = s32; id1 = id; l1 = l; bits1 = ((uint64_t)hi << 32) | lo;
+      } else {
+        t2 = fmaxf(t2, s32);
+      }
+    };
+    // A wave whose kept tokens are few and scattered takes each lane's own next
+    // token per step: the steps are the most tokens a lane holds, where the
+    // pair loop takes one for every pair some lane holds (64 x 151936 f32 under
+    // the serving rules with 2048 history IDs, per call: 51.1 -> 48.4 us).
+    const uint32_t held = wave_max_u32((uint32_t)__builtin_popcount(mine));
+    const uint32_t pairs = (uint32_t)__builtin_popcount(wave_or_u32((mine | (mine >> 1)) & 0x55555555u));
+    if (held < pairs) {
+      for (uint32_t r = mine; r; r &= r - 1u) {
+        const uint32_t bt = (uint32_t)__builtin_ctz(r), id = id0 + 2u * RNT * (bt >> 1) + (bt & 1u);
+        const float l = adjust(id, Quad<In>::one(lrow + id));
+        const uint64_t bits = race_bits(seed, choice, position, id);
+        score(id, l, (uint32_t)(bits >> 32), (uint32_t)bits);
+      }
+    } else
     // four pairs' logits in flight per thread
 #pragma unroll
     for (uint32_t q = 0; q < RPT / 8u; ++q) {
@@ -370,17 +404,8 @@ __global__ __launch_bounds__(RNT) void race_kernel(RaceArgs A) {
         uint32_t c4[4] = {id >> 1, position, choice, 0x72616365u};
         philox4x32_10(c4, (uint32_t)seed, (uint32_t)(seed >> 32));
 #pragma unroll
-        for (uint32_t e = 0; e < 2u; ++e) {
-          if (!((kb >> e) & 1u)) continue;
-          const float l = pl[j][e];
-          mass += expo(((double)l - (double)m) * invT);   // (within ulps of the quotient: the mass feeds only the logprob)
-          const float s32 = (l - m) * invT32 + gumbel32(c4[2u * e], c4[2u * e + 1u]);
-          if (s32 > t1) {
-            t2 = t1; t1 = s32; id1 = id + e; l1 = l; bits1 = ((uint64_t)c4[2u * e] << 32) | c4[2u * e + 1u];
-          } else {
-            t2 = fmaxf(t2, s32);
-          }
-        }
+        for (uint32_t e = 0; e < 2u; ++e)
+          if ((kb >> e) & 1u) score(id + e, pl[j][e], c4[2u * e], c4[2u * e + 1u]);
       }
     }
     float smax = t1;
@@ -548,7 +573,9 @@ extern "C" int mxs_sample_race(mxs_ctx* ctx, const mxs_batch* b, const mxs_race*
   A.rows = b->rows;
   A.V = b->vocab;
   A.nwords = (b->vocab + 31u) / 32u;
-  A.C = (b->vocab + mxs::RT - 1u) / mxs::RT;
+  auto chunks = [&](uint32_t rpt) { return (b->vocab + mxs::RNT * rpt - 1u) / (mxs::RNT * rpt); };
+  const bool wide = (uint64_t)b->rows * chunks(mxs::RPT_SHORT) > mxs::RWIDE;
+  A.C = chunks(wide ? mxs::RPT_WIDE : mxs::RPT_SHORT);
   A.temperature = b->temperature;
   A.rep = b->repetition ? b->repetition : ctx->d_one_f32;
   A.pres = b->presence ? b->presence : ctx->d_zero_f32;
@@ -572,10 +599,10 @@ extern "C" int mxs_sample_race(mxs_ctx* ctx, const mxs_batch* b, const mxs_race*
   (void)hipGetDevice(&prev);
   if (prev != ctx->device) (void)hipSetDevice(ctx->device);
   const dim3 grid(A.C * b->rows);   // (row, chunk) order
-  if (b->dtype == MXS_F32)
-    hipLaunchKernelGGL(mxs::race_kernel<float>, grid, dim3(mxs::RNT), 0, ctx->stream, A);
-  else
-    hipLaunchKernelGGL(mxs::race_kernel<uint16_t>, grid, dim3(mxs::RNT), 0, ctx->stream, A);
+  void (*kernel)(mxs::RaceArgs) =
+      b->dtype == MXS_F32 ? (wide ? mxs::race_kernel<float, mxs::RPT_WIDE> : mxs::race_kernel<float, mxs::RPT_SHORT>)
+                          : (wide ? mxs::race_kernel<uint16_t, mxs::RPT_WIDE> : mxs::race_kernel<uint16_t, mxs::RPT_SHORT>);
+  hipLaunchKernelGGL(kernel, grid, dim3(mxs::RNT), 0, ctx->stream, A);
   hipError_t e = hipGetLastError();
   if (prev != ctx->device) (void)hipSetDevice(prev);
   if (e != hipSuccess) return hip_fail(ctx, e, "race_kernel launch");

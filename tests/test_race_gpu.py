@@ -205,3 +205,36 @@ def test_race_heavy_histories(torch_mod, sampler, orc):
     b.history_ids = np.concatenate(hists)
     gpu, _ = check(torch_mod, sampler, orc, b, 17)
     assert (gpu["status"] == 0).all(), gpu["status"]
+
+
+# Pair and chunk edges of the race kernel: odd and ragged vocabularies (a pair's
+# second token past the row), vocabularies around its 4096- and 8192-token
+# chunks, and batches on both sides of the rule that picks between them
+# (rows x ceil(vocab / 4096) > 4096), with whole-row races, flat top-p rows
+# (finished over the whole row), small kept sets and histories in each.
+@pytest.mark.parametrize("rows,vocab,bf16", [(8, 1, False), (8, 3, False), (16, 4095, True), (16, 4097, False), (16, 8193, True),
+                                             (16, 20479, False), (24, 50257, True), (40, 40003, False), (600, 28673, False),
+                                             (1100, 12289, True)])
+def test_race_edges(torch_mod, orc, rows, vocab, bf16):
+    from metallix_amd import Sampler, synth
+
+    s = synth.Stream(rows * 1000 + vocab)
+    x = (2.0 * s.normal(rows * vocab)).reshape(rows, vocab).astype(np.float32)
+    bits = None
+    if bf16:
+        bits = synth.to_bf16_bits(x)
+        x = synth.bf16_bits_to_f32(bits)
+    r = np.arange(rows)
+    b = synth.Batch(name="race-edges", logits=x, temperature=0.6 + 0.1 * (r % 7), uniform=np.zeros(rows), bf16_bits=bits)
+    b.top_k = np.where(r % 4 == 1, 20, 0).astype(np.uint32)
+    b.top_p = np.where(r % 4 == 2, 0.9, 1.0)
+    b.min_p = np.where(r % 4 == 3, 0.05, 0.0)
+    b.history_offsets = (np.minimum(r.tolist() + [rows], rows // 2) * 50).astype(np.uint32)   # the first half of the rows
+    b.history_ids = (s.u64(rows // 2 * 50) % np.uint64(vocab)).astype(np.uint32)
+    b.repetition = np.full(rows, 1.1, dtype=np.float32)
+    b.presence = np.full(rows, 0.2, dtype=np.float32)
+    b.frequency = np.full(rows, 0.1, dtype=np.float32)
+    sampler = Sampler(max_rows=rows, max_vocab=vocab)
+    gpu, _ = check(torch_mod, sampler, orc, b, 19)
+    assert (gpu["status"] == 0).all()
+    sampler.close()
