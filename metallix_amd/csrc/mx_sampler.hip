@@ -2993,9 +2993,7 @@ __device__ __forceinline__ bool finish_w1(const FinCtx& X, FinSmem& F) {
   } else if (c.top_p < 1.0) {
     // the reference walks the tokens whose weight reaches 1e-9 of the total:
     // every min-p member must clear that level
-    // (a nuc row's cut is known to lie among its candidates; below the 1e-9
-    // level the reference falls back to the whole row, the same prefix)
-    if (!X.nuc && !(c.min_p * (1.0 - 1e-12) > 1e-9 * (X.total + X.total_err) * (1.0 + 1e-12))) return false;
+    if (!(c.min_p * (1.0 - 1e-12) > 1e-9 * (X.total + X.total_err) * (1.0 + 1e-12))) return false;
     theta_set = true;
     theta = c.top_p * X.total;
     theta_err = c.top_p * X.total_err + U * theta;
@@ -3592,9 +3590,10 @@ __device__ __forceinline__ bool finish_row(const SampleArgs& A, FinSmem& F, cons
   };
   // A nuc row: the nucleus lies among the candidates every chunk lists in
   // full (those from the largest chunk threshold up) when their mass reaches
-  // top_p of the row's.  f32 weights: relative error below 1e-5 (three
-  // roundings of an exponent of at most 126 octaves and 2 ulp of exp2); a
-  // mass within 4e-5 of the bar counts as below it.
+  // top_p of the row's.  f32 weights: three roundings (2^-24 each) of an
+  // exponent of at most 126 octaves make 126 ln 2 3 2^-24 = 1.56e-5, the exp2
+  // and the FR-term f32 sum 5e-7 more, so the relative error stays below
+  // 1.7e-5; a mass within 4e-5 of the bar counts as below it.
   if (nuc && !X.lds_c) return true;
   const bool short_row = ((mode == M_TOPK && c.k <= 64u) || mode == M_MINP) && ncand > 0u &&
                          ncand <= (uint32_t)(WR * 64) && X.lds_c;
