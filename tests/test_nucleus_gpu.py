@@ -232,3 +232,39 @@ def test_export_of_top_p_rows(torch_mod, orc, opt):
             elif width == V:
                 assert np.isin(np.nonzero(ref["kept"][r])[0], i).all()
     s.close()
+
+
+def crowded(rng, R, V, levels):
+    """N(0, 0.3^2), or two levels whose second is spread over a few thousand ulps."""
+    if not levels:
+        return (0.3 * rng.standard_normal((R, V))).astype(np.float32)
+    x = (np.float32(1.0) + rng.integers(0, 4000, (R, V)).astype(np.float32) * np.float32(2.0 ** -23)).astype(np.float32)
+    top = rng.random((R, V)) < 0.02
+    return np.where(top, np.float32(4.0) + rng.standard_normal((R, V)).astype(np.float32) * np.float32(0.1), x).astype(np.float32)
+
+
+# Cuts inside a mass bin (1/64 octave) that holds more than the 4096 tokens the
+# whole-row finish sorts, at distinct keys: N(0, 0.3^2) at T 4 to 20 puts V / 100
+# tokens and more in a bin; the second level of the two-level rows is one bin.
+# top_p cuts far from the f64 sums' error bound (1e-11 of the row): status 0, the
+# exact kept set.
+@pytest.mark.parametrize("levels,bf16,history", [(False, False, 0), (False, True, 0), (False, False, 300), (True, False, 0),
+                                                 (True, False, 300)])
+@pytest.mark.parametrize("V", [151936, 262144])
+def test_crowded_distinct_keys(torch_mod, orc, V, levels, bf16, history):
+    from metallix_amd import Sampler
+    from metallix_amd.synth import bf16_bits_to_f32, to_bf16_bits
+
+    R = 4
+    b = batch("flat", R, V, bf16=bf16, history=history, seed=13)
+    b.logits = crowded(np.random.default_rng([V, levels, bf16]), R, V, levels)
+    if bf16:
+        b.bf16_bits = to_bf16_bits(b.logits)
+        b.logits = bf16_bits_to_f32(b.bf16_bits)
+    b.temperature, b.top_p = np.array([4.0, 8.0, 20.0, 5.0]), np.array([0.3, 0.5, 0.9, 0.7])
+    print(f"case nucleus crowded vocab {V} levels {levels} bf16 {bf16} history {history}", flush=True)
+    s = Sampler(max_rows=R, max_vocab=V)
+    gpu = run_gpu(torch_mod, s, b)
+    assert (gpu["status"] == 0).all(), gpu["status"]
+    compare(b, gpu, orc.sample_batch(b, debug=True))
+    s.close()

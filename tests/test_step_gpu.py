@@ -132,6 +132,33 @@ def test_step_bf16_masked_rows(torch_mod, sampler, orc):
     check_step(torch_mod, sampler, orc, b, sup, tops, 64)
 
 
+@pytest.mark.parametrize("V,bf16,history", [(40003, False, 0), (151936, True, 0), (40003, False, 200)])
+def test_step_flat_top_p_rows(torch_mod, sampler, orc, V, bf16, history):
+    """Receipts beside top-p rows without a top-k that are finished over their
+    whole row (flat: the nucleus is most of it), next to rows of other rules."""
+    from metallix_amd import synth
+
+    R = 6
+    s = synth.Stream(V + history)
+    x = s.normal(R * V).reshape(R, V).astype(np.float32)
+    bits = synth.to_bf16_bits(x) if bf16 else None
+    if bf16:
+        x = synth.bf16_bits_to_f32(bits)
+    b = synth.Batch(name="step-flat", logits=x, temperature=np.full(R, 0.9), uniform=s.uniform(R), bf16_bits=bits)
+    b.top_p = np.array([0.95, 0.9, 1.0, 0.8, 0.95, 0.99])
+    b.top_k = np.array([0, 0, 20, 0, 1000, 0], dtype=np.uint32)
+    if history:
+        b.history_offsets = (np.arange(R + 1) * history).astype(np.uint32)
+        b.history_ids = (s.u64(R * history) % np.uint64(V)).astype(np.uint32)
+        b.repetition = np.full(R, 1.1, dtype=np.float32)
+        b.presence = np.full(R, 0.2, dtype=np.float32)
+        b.frequency = np.full(R, 0.1, dtype=np.float32)
+    sup = [3, V - 2]
+    b = suppressed(b, sup)
+    tops = np.array([20, 0, 5, NONE, 20, 1], dtype=np.uint32)
+    check_step(torch_mod, sampler, orc, b, sup, tops, 28)
+
+
 def test_step_receipt_ties_flat_and_nonfinite(torch_mod, sampler, orc):
     """Receipt edge cases of the one-pass step: a constant row and a top
     plateau of 3000 equal logits (ties past the chunks' candidate capacity:
