@@ -6318,7 +6318,14 @@ __global__ __launch_bounds__(NT) void sample_kernel(
   const uint32_t mode = chunk_mode(c, V);
   // a step receipt for this row (mxs_step)
   const bool rx = RX && A.rx_want[row] != MXS_RECEIPT_NONE;
-  const bool nuc = !c.err && nucleus_only(c, V);
+  // (asked again at each use in the bf16 receipt kernel: kept across its bodies,
+  // the answer made them spill 12 more vector registers, and a step of 12 rows
+  // took 4 to 9% longer; the other instantiations are the better for keeping it)
+  const bool nuc0 = !c.err && nucleus_only(c, V);
+  auto is_nuc = [&]() {
+    if constexpr (RX && sizeof(In) == 2) return !c.err && nucleus_only(c, V);
+    else return nuc0;
+  };
   uint32_t rxw;   // the receipt work left after the body
   {
     const uint32_t hn = c.he > c.hb ? c.he - c.hb : 0u, bn = c.be > c.bb ? c.be - c.bb : 0u;
@@ -6345,7 +6352,7 @@ __global__ __launch_bounds__(NT) void sample_kernel(
         else rxw = chunk_fast<In, M_MINP, false, RX>(A, U, c, row, chunk, c0, c1, 0u, 0u, rx);
       }
     } else {
-      if (nuc) {
+      if (is_nuc()) {
         nuc_chunk<In>(U, row, chunk);
         rxw = rx ? RX_FULL : 0u;
       } else {
@@ -6390,7 +6397,7 @@ __global__ __launch_bounds__(NT) void sample_kernel(
     return;
   }
   stamp(A, row, MAXC, 0);
-  if (nuc) {
+  if (is_nuc()) {
     nuc_finish<In>(U.f, row);
   } else {
     FinLoads P;
